@@ -183,9 +183,10 @@ int sfft_plan_get_info(sfft_plan plan, sfft_plan_info *info) {
         info->n = p.n();
         info->kind = p.kind();
         info->precision = p.prec();
-        // a chirp-z plan reports the layout of its length-M inner FFT (run twice)
+        // a chirp-z plan reports the layout of a length-M FFT (run twice, or
+        // once over HBM where both run in one launch)
         const sfft::Plan &q = p.bluestein() ? *p.bluestein_inner() : p;
-        info->passes = (int)q.passes().size() * (p.bluestein() ? 2 : 1);
+        info->passes = p.bluestein_fused() ? 1 : (int)q.passes().size() * (p.bluestein() ? 2 : 1);
         info->chirp_length = p.bluestein_m();
         const sfft::PassDesc &pd = q.passes()[0].pd;
         info->nradices = pd.nstages;

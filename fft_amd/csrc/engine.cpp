@@ -430,7 +430,11 @@ Plan::Plan(size_t n, int kind, int prec, const PlanHints *h) : n_(n), kind_(kind
                         "16-bit storage and F32X: only lengths with factors 2, 3, 5, 7, 11, 13");
         if (cn_ > kMaxBluestein)
             throw Error(SFFT_ERR_UNSUPPORTED_SIZE, "size " + std::to_string(n) + " too large");
-        bs_m_ = bluestein_length(cn_);
+        // one launch where a compiled convolution length fits LDS; the
+        // launch sequence otherwise
+        bs_row_ = bluestein_length(cn_);
+        chirp_ = find_chirp(cn_, prec == kF64 ? 1 : 0);
+        bs_m_ = chirp_ ? (size_t)chirp_->m : bs_row_;
         try {
             bs_inner_.reset(new Plan(bs_m_, kC2C, prec));
         } catch (const Error &e) {
@@ -619,7 +623,61 @@ void Plan::build_bluestein() {
               "chirp generation");
     bs_inner_->execute(tmp, bs_m_, d_bhat_, bs_m_, 1, 0, nullptr);
     check_hip(bs_scale<T>((C2<T> *)d_bhat_, bs_m_, 1.0 / (double)bs_m_, nullptr), "chirp scale");
+    if (chirp_) {
+        // stage twiddles of the kernel's radices, taken forwards and backwards
+        std::vector<int> rs(chirp_->radices, chirp_->radices + chirp_->nst);
+        const std::vector<int> back(rs.rbegin(), rs.rend());
+        auto count = [](const std::vector<int> &r) {
+            size_t c = 0, ns = 1;
+            for (int x : r) {
+                if (ns > 1) c += ns * tw_group(x);
+                ns *= x;
+            }
+            return c;
+        };
+        chirp_twb_ = rs == back ? 0 : count(rs);
+        const size_t total = chirp_twb_ + count(back);
+        alloc(&d_tw_, total * eb);
+        table_bytes_ += total * eb;
+        auto fill = [&](const std::vector<int> &r, size_t off) {
+            size_t ns = 1;
+            for (int x : r) {
+                if (ns > 1) {
+                    check_hip(gen_stage_twiddles<T>((C2<T> *)d_tw_, (int)off, (int)ns, x, nullptr),
+                              "twiddle generation");
+                    off += ns * tw_group(x);
+                }
+                ns *= x;
+            }
+        };
+        fill(rs, 0);
+        if (chirp_twb_) fill(back, chirp_twb_);
+    }
     check_hip(hipDeviceSynchronize(), "chirp tables");
+}
+
+// The chirp-z transform of a short length in one launch.
+template <typename T>
+void Plan::run_chirp(const void *in, int64_t din, void *out, int64_t dout, size_t batch,
+                     int inverse, hipStream_t stream) const {
+    ChirpArgs<T> a{};
+    a.in = (const C2<T> *)in;
+    a.out = (C2<T> *)out;
+    a.in_dist = din;
+    a.out_dist = dout;
+    a.w = (const C2<T> *)d_chirp_;
+    a.bhat = (const C2<T> *)d_bhat_;
+    a.twf = (const C2<T> *)d_tw_;
+    a.twb = a.twf + chirp_twb_;
+    a.real_tw = (const C2<T> *)d_real_tw_;
+    a.rot = (const C2<T> *)d_rot_;
+    a.n = (int32_t)cn_;
+    a.batch = (int32_t)batch;
+    a.mode = kind_ == kC2C ? kModeC2C : (inverse ? kModeC2R : kModeR2C);
+    a.inverse = inverse;
+    a.half_shift = kind_ == kR2CHalf;
+    const unsigned grid = (unsigned)((batch + chirp_->tpw - 1) / chirp_->tpw);
+    check_hip(chirp_->launch(&a, grid, stream), "chirp-z launch");
 }
 
 template <typename T>
@@ -802,6 +860,10 @@ void Plan::run(const void *in, size_t in_dist, void *out, size_t out_dist, size_
             din = (int64_t)(in_dist / 2);
         }
     }
+    if (chirp_) {
+        run_chirp<T>(in, din, out, dout, batch, inverse, stream);
+        return;
+    }
     if (bs_inner_) {
         run_bluestein<T>(in, din, out, dout, batch, inverse, stream, ws);
         return;
@@ -953,7 +1015,7 @@ template void Plan::run_fixed<double>(const void *, void *, size_t, int, hipStre
 
 size_t Plan::workspace_bytes(size_t batch, bool in_place) const {
     const size_t cb = 2 * real_bytes(prec_);  // one complex value in HBM
-    if (bs_inner_) return 2 * bs_m_ * cb * batch;
+    if (bs_inner_) return 2 * bs_row_ * cb * batch;
     if (in_place && passes_.size() > 1) return cn_ * cb * batch;
     return 0;
 }
@@ -978,7 +1040,7 @@ void Plan::execute(const void *in, size_t in_dist, void *out, size_t out_dist, s
         throw Error(SFFT_ERR_ALIASING, "input and output overlap other than exactly in place");
     if (in_dist < default_in_dist(inverse) || out_dist < default_out_dist(inverse))
         throw Error(SFFT_ERR_INVALID_ARG, "batch distance shorter than one transform");
-    if (bs_inner_ && batch > (0x7fffffffull / bs_m_))
+    if (bs_inner_ && batch > (0x7fffffffull / bs_row_))
         throw Error(SFFT_ERR_INVALID_ARG, "batch too large");
     const size_t need = workspace_bytes(batch, in_place);
     struct Owned {
@@ -995,7 +1057,7 @@ void Plan::execute(const void *in, size_t in_dist, void *out, size_t out_dist, s
         const uintptr_t w0 = (uintptr_t)ws;
         if ((w0 < i0 + in_len && i0 < w0 + need) || (w0 < o0 + out_len && o0 < w0 + need))
             throw Error(SFFT_ERR_ALIASING, "workspace overlaps the input or the output");
-    } else if (need) {
+    } else if (need && !chirp_) {
         if (hipMallocAsync(&owned.p, need, stream) != hipSuccess) {
             (void)hipGetLastError();
             owned.p = nullptr;

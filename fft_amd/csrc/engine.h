@@ -11,6 +11,7 @@
 #include <string>
 #include <vector>
 
+#include "chirp.h"
 #include "fixed.h"
 #include "kernels.h"
 #include "plan_desc.h"
@@ -97,15 +98,19 @@ class Plan {
     // plans read each transform whole before writing it; two-pass plans run
     // in place through a workspace for the intermediate.
     bool in_place_direct() const { return bs_inner_ != nullptr || passes_.size() == 1; }
-    // Device workspace an execute call of `batch` transforms needs: chirp-z
-    // rows (2 M values per transform) or, in place on a two-pass length, the
-    // intermediate (cn values per transform); 0 if none.
+    // Device workspace to hand to an execute call of `batch` transforms:
+    // chirp-z rows (2 M values per transform, M the smallest 2^a 3^b 5^c
+    // convolution length; lengths that run in one launch leave it untouched)
+    // or, in place on a two-pass length, the intermediate (cn values per
+    // transform); 0 if none.
     size_t workspace_bytes(size_t batch, bool in_place) const;
     // Chirp-z plan: the length has a prime factor the kernels do not plan;
     // the transform runs as a convolution through FFTs of length bluestein_m().
     bool bluestein() const { return bs_inner_ != nullptr; }
     size_t bluestein_m() const { return bs_m_; }
     const Plan *bluestein_inner() const { return bs_inner_.get(); }
+    // ... in one launch, which needs no workspace (chirp.h)
+    bool bluestein_fused() const { return chirp_ != nullptr; }
 
     // in/out: device pointers; dists in elements of the in/out type
     // (complex for C2C, real/complex for the real kinds).  ws / ws_bytes: a
@@ -147,6 +152,9 @@ class Plan {
     template <typename T>
     void build_bluestein();
     template <typename T>
+    void run_chirp(const void *in, int64_t din, void *out, int64_t dout, size_t batch,
+                   int inverse, hipStream_t stream) const;
+    template <typename T>
     void run_bluestein(const void *in, int64_t din, void *out, int64_t dout, size_t batch,
                        int inverse, hipStream_t stream, void *ws) const;
 
@@ -166,6 +174,9 @@ class Plan {
     size_t table_bytes_ = 0;
     std::unique_ptr<Plan> bs_inner_;
     size_t bs_m_ = 0;
+    size_t bs_row_ = 0;  // values per workspace row of the launch sequence
+    const ChirpKernel *chirp_ = nullptr;  // the one-launch kernel, if any
+    size_t chirp_twb_ = 0;                // its second FFT's twiddles in d_tw_
     void *d_chirp_ = nullptr;
     void *d_bhat_ = nullptr;
 };

@@ -1,7 +1,9 @@
-// fixed_registry.cpp -- lookup table of the compiled fixed-plan kernels.
+// fixed_registry.cpp -- lookup tables of the compiled fixed-plan and chirp-z
+// kernels.
 #include <mutex>
 #include <vector>
 
+#include "chirp.h"
 #include "fixed.h"
 
 namespace sfft {
@@ -34,6 +36,24 @@ int fixed_variant_count(int n, int prec, int real) {
     for (const auto &k : registry())
         if (k.n == n && k.prec == prec && k.real == real) ++c;
     return c;
+}
+
+static std::vector<ChirpKernel> &chirp_registry() {
+    static std::vector<ChirpKernel> r;
+    return r;
+}
+
+void register_chirp(const ChirpKernel &k) {
+    std::lock_guard<std::mutex> lock(registry_mutex());
+    chirp_registry().push_back(k);
+}
+
+const ChirpKernel *find_chirp(size_t n, int prec) {
+    std::lock_guard<std::mutex> lock(registry_mutex());
+    const ChirpKernel *best = nullptr;
+    for (const auto &k : chirp_registry())
+        if (k.prec == prec && (size_t)k.m + 1 >= 2 * n && (!best || k.m < best->m)) best = &k;
+    return best;
 }
 
 }  // namespace sfft
