@@ -45,6 +45,14 @@ __global__ void k_bs_scale(C2<T> *z, uint64_t m_len, T s) {
         z[m] = {z[m].x * s, z[m].y * s};
 }
 
+template <typename T>
+__global__ void k_bs_digit_swap(const C2<T> *src, C2<T> *dst, uint64_t n1, uint64_t m_len) {
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    const uint64_t n2 = m_len / n1;
+    for (uint64_t m = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; m < m_len; m += stride)
+        dst[m] = src[m / n2 + n1 * (m % n2)];
+}
+
 // a[b][m] = load(x[b], m) * w[m] for m < N, 0 up to M.  The load applies the
 // conjugation of the inverse, the half-bin rotation of a forward
 // ModifiedRealFFT, or the real inverse pre-process of bin m.
@@ -130,6 +138,14 @@ hipError_t bs_scale(C2<T> *z, size_t m_len, double s, hipStream_t stream) {
 }
 
 template <typename T>
+hipError_t bs_digit_swap(const C2<T> *src, C2<T> *dst, size_t n1, size_t m_len,
+                         hipStream_t stream) {
+    hipLaunchKernelGGL((k_bs_digit_swap<T>), grid_1d(m_len), dim3(256), 0, stream, src, dst,
+                       (uint64_t)n1, (uint64_t)m_len);
+    return hipGetLastError();
+}
+
+template <typename T>
 hipError_t bs_pre(const C2<T> *in, int64_t in_dist, C2<T> *a, size_t m_len, size_t n_len,
                   size_t batch, const C2<T> *w, int mode, int conj_in, int half_shift,
                   const C2<T> *tmi, const C2<T> *rot, hipStream_t stream) {
@@ -159,6 +175,7 @@ hipError_t bs_post(const C2<T> *c, size_t m_len, C2<T> *out, int64_t out_dist, s
 #define SFFT_BS_INSTANTIATE(T)                                                                  \
     template hipError_t bs_gen_chirp<T>(C2<T> *, C2<T> *, size_t, size_t, hipStream_t);       \
     template hipError_t bs_scale<T>(C2<T> *, size_t, double, hipStream_t);                    \
+    template hipError_t bs_digit_swap<T>(const C2<T> *, C2<T> *, size_t, size_t, hipStream_t); \
     template hipError_t bs_pre<T>(const C2<T> *, int64_t, C2<T> *, size_t, size_t, size_t,    \
                                   const C2<T> *, int, int, int, const C2<T> *, const C2<T> *, \
                                   hipStream_t);                                               \

@@ -1,0 +1,41 @@
+// chirp_split.hip -- the kernels of chirp-z transforms in three launches:
+// columns of N1 = 16 b (ChirpColReg<type, columns per block, radices>: 256-byte
+// rows) and rows of N2, a power of two (ChirpReg<type, true, N2, threads per
+// row, rows per block, minimum waves per SIMD, radices...>).  The lengths
+// M = 16 b N2 are 6 to 15 percent apart.
+#include "chirp.h"
+
+namespace sfft {
+namespace {
+const ChirpColReg<float, 32, 16, 8> c128;
+const ChirpColReg<float, 32, 16, 9> c144;
+const ChirpColReg<float, 32, 16, 10> c160;
+const ChirpColReg<float, 32, 16, 11> c176;
+const ChirpColReg<float, 32, 16, 12> c192;
+const ChirpColReg<float, 32, 16, 13> c208;
+const ChirpColReg<float, 32, 16, 15> c240;
+const ChirpColReg<double, 16, 16, 8> d128;
+const ChirpColReg<double, 16, 16, 9> d144;
+const ChirpColReg<double, 16, 16, 10> d160;
+const ChirpColReg<double, 16, 16, 11> d176;
+const ChirpColReg<double, 16, 16, 12> d192;
+const ChirpColReg<double, 16, 16, 13> d208;
+const ChirpColReg<double, 16, 16, 15> d240;
+const ChirpReg<float, true, 128, 16, 16, 4, 8, 2, 8> r128;
+const ChirpReg<float, true, 256, 16, 16, 4, 16, 16> r256;
+const ChirpReg<float, true, 512, 64, 4, 4, 8, 8, 8> r512;
+const ChirpReg<float, true, 1024, 64, 4, 4, 16, 4, 16> r1024;
+const ChirpReg<float, true, 2048, 128, 2, 4, 16, 8, 16> r2048;
+const ChirpReg<float, true, 4096, 256, 1, 4, 16, 16, 16> r4096;
+const ChirpReg<float, true, 8192, 512, 1, 4, 16, 8, 4, 16> r8192;
+const ChirpReg<float, true, 16384, 1024, 1, 4, 16, 16, 4, 16> r16384;
+const ChirpReg<double, true, 64, 8, 16, 2, 8, 8> s64;
+const ChirpReg<double, true, 128, 16, 8, 2, 8, 2, 8> s128;
+const ChirpReg<double, true, 256, 16, 8, 2, 16, 16> s256;
+const ChirpReg<double, true, 512, 64, 2, 2, 8, 8, 8> s512;
+const ChirpReg<double, true, 1024, 64, 2, 2, 16, 4, 16> s1024;
+const ChirpReg<double, true, 2048, 128, 1, 2, 16, 8, 16> s2048;
+const ChirpReg<double, true, 4096, 256, 1, 2, 16, 16, 16> s4096;
+const ChirpReg<double, true, 8192, 512, 1, 2, 16, 8, 4, 16> s8192;
+}  // namespace
+}  // namespace sfft

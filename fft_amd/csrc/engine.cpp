@@ -430,11 +430,14 @@ Plan::Plan(size_t n, int kind, int prec, const PlanHints *h) : n_(n), kind_(kind
                         "16-bit storage and F32X: only lengths with factors 2, 3, 5, 7, 11, 13");
         if (cn_ > kMaxBluestein)
             throw Error(SFFT_ERR_UNSUPPORTED_SIZE, "size " + std::to_string(n) + " too large");
-        // one launch where a compiled convolution length fits LDS; the
-        // launch sequence otherwise
+        // one launch where a compiled convolution length fits LDS, three
+        // where it is a compiled column length times a compiled row length
+        // (100003 x 64, both directions: 639 us as the launch sequence, 292 us), the launch
+        // sequence beyond (M above 240 x 16384 in F32, 240 x 8192 in F64)
         bs_row_ = bluestein_length(cn_);
         chirp_ = find_chirp(cn_, prec == kF64 ? 1 : 0);
-        bs_m_ = chirp_ ? (size_t)chirp_->m : bs_row_;
+        if (!chirp_) find_chirp_split(cn_, prec == kF64 ? 1 : 0, chirp_cols_, chirp_);
+        bs_m_ = !chirp_ ? bs_row_ : (size_t)chirp_->m * (size_t)(chirp_cols_ ? chirp_cols_->m : 1);
         try {
             bs_inner_.reset(new Plan(bs_m_, kC2C, prec));
         } catch (const Error &e) {
@@ -636,7 +639,10 @@ void Plan::build_bluestein() {
             return c;
         };
         chirp_twb_ = rs == back ? 0 : count(rs);
-        const size_t total = chirp_twb_ + count(back);
+        chirp_twc_ = chirp_twb_ + count(back);
+        std::vector<int> cs;
+        if (chirp_cols_) cs.assign(chirp_cols_->radices, chirp_cols_->radices + chirp_cols_->nst);
+        const size_t total = chirp_twc_ + count(cs);
         alloc(&d_tw_, total * eb);
         table_bytes_ += total * eb;
         auto fill = [&](const std::vector<int> &r, size_t off) {
@@ -652,32 +658,78 @@ void Plan::build_bluestein() {
         };
         fill(rs, 0);
         if (chirp_twb_) fill(back, chirp_twb_);
+        fill(cs, chirp_twc_);
+    }
+    if (chirp_cols_) {
+        // the rows' order of the transformed kernel, and their twiddles
+        const size_t n1 = (size_t)chirp_cols_->m, n2 = (size_t)chirp_->m;
+        alloc(&d_twist_, bs_m_ * eb);
+        table_bytes_ += bs_m_ * eb;
+        check_hip(gen_post_twiddles_full<T>((C2<T> *)d_twist_, n2, bs_m_, nullptr),
+                  "twiddle generation");
+        check_hip(bs_digit_swap<T>((const C2<T> *)d_bhat_, (C2<T> *)tmp, n1, bs_m_, nullptr),
+                  "chirp order");
+        check_hip(hipMemcpyAsync(d_bhat_, tmp, bs_m_ * eb, hipMemcpyDeviceToDevice, nullptr),
+                  "chirp order");
     }
     check_hip(hipDeviceSynchronize(), "chirp tables");
 }
 
-// The chirp-z transform of a short length in one launch.
+// The chirp-z transform in one launch, or in three over ws.
 template <typename T>
 void Plan::run_chirp(const void *in, int64_t din, void *out, int64_t dout, size_t batch,
-                     int inverse, hipStream_t stream) const {
+                     int inverse, hipStream_t stream, void *ws) const {
+    const int mode = kind_ == kC2C ? kModeC2C : (inverse ? kModeC2R : kModeR2C);
+    const C2<T> *tw = (const C2<T> *)d_tw_;
+    ChirpColArgs<T> c{};
+    if (chirp_cols_) {
+        c.in = (const C2<T> *)in;
+        c.out = (C2<T> *)ws;
+        c.in_dist = din;
+        c.out_dist = (int64_t)bs_m_;
+        c.w = (const C2<T> *)d_chirp_;
+        c.tw = tw + chirp_twc_;
+        c.real_tw = (const C2<T> *)d_real_tw_;
+        c.rot = (const C2<T> *)d_rot_;
+        c.tiles = make_fastdiv((uint32_t)(chirp_->m / chirp_cols_->tpw));
+        c.n = (int32_t)cn_;
+        c.n2 = (int32_t)chirp_->m;
+        c.mode = mode;
+        c.inverse = inverse;
+        c.half_shift = kind_ == kR2CHalf;
+        check_hip(chirp_cols_->launch(&c, 0, (unsigned)(batch * c.tiles.d), stream),
+                  "chirp-z columns launch");
+    }
     ChirpArgs<T> a{};
-    a.in = (const C2<T> *)in;
-    a.out = (C2<T> *)out;
-    a.in_dist = din;
-    a.out_dist = dout;
-    a.w = (const C2<T> *)d_chirp_;
+    a.in = (const C2<T> *)(chirp_cols_ ? ws : in);
+    a.out = (C2<T> *)(chirp_cols_ ? ws : out);
+    a.in_dist = chirp_cols_ ? (int64_t)chirp_->m : din;
+    a.out_dist = chirp_cols_ ? (int64_t)chirp_->m : dout;
+    a.w = (const C2<T> *)(chirp_cols_ ? d_twist_ : d_chirp_);
     a.bhat = (const C2<T> *)d_bhat_;
-    a.twf = (const C2<T> *)d_tw_;
-    a.twb = a.twf + chirp_twb_;
+    a.twf = tw;
+    a.twb = tw + chirp_twb_;
     a.real_tw = (const C2<T> *)d_real_tw_;
     a.rot = (const C2<T> *)d_rot_;
     a.n = (int32_t)cn_;
-    a.batch = (int32_t)batch;
-    a.mode = kind_ == kC2C ? kModeC2C : (inverse ? kModeC2R : kModeR2C);
+    a.rows = chirp_cols_ ? chirp_cols_->m : 1;
+    a.batch = (int32_t)(batch * (size_t)a.rows);
+    a.mode = mode;
     a.inverse = inverse;
     a.half_shift = kind_ == kR2CHalf;
-    const unsigned grid = (unsigned)((batch + chirp_->tpw - 1) / chirp_->tpw);
-    check_hip(chirp_->launch(&a, grid, stream), "chirp-z launch");
+    const unsigned grid = (unsigned)(((size_t)a.batch + chirp_->tpw - 1) / chirp_->tpw);
+    check_hip(chirp_->launch(&a, 0, grid, stream), "chirp-z launch");
+    if (!chirp_cols_) return;
+    c.in = (const C2<T> *)ws;
+    c.out = (C2<T> *)out;
+    c.in_dist = (int64_t)bs_m_;
+    c.out_dist = dout;
+    check_hip(chirp_cols_->launch(&c, 1, (unsigned)(batch * c.tiles.d), stream),
+              "chirp-z columns launch");
+    if (kind_ != kC2C && !inverse)
+        check_hip(launch_real_post<T>((C2<T> *)out, dout, (int)cn_, batch,
+                                      (const C2<T> *)d_real_tw_, kind_ == kR2CHalf, stream),
+                  "real post-process launch");
 }
 
 template <typename T>
@@ -708,6 +760,7 @@ void Plan::run_bluestein(const void *in, int64_t din, void *out, int64_t dout, s
 Plan::~Plan() {
     if (d_chirp_) (void)hipFree(d_chirp_);
     if (d_bhat_) (void)hipFree(d_bhat_);
+    if (d_twist_) (void)hipFree(d_twist_);
     if (d_tw_) (void)hipFree(d_tw_);
     if (d_real_tw_) (void)hipFree(d_real_tw_);
     if (d_rot_) (void)hipFree(d_rot_);
@@ -861,7 +914,7 @@ void Plan::run(const void *in, size_t in_dist, void *out, size_t out_dist, size_
         }
     }
     if (chirp_) {
-        run_chirp<T>(in, din, out, dout, batch, inverse, stream);
+        run_chirp<T>(in, din, out, dout, batch, inverse, stream, ws);
         return;
     }
     if (bs_inner_) {
@@ -1020,6 +1073,11 @@ size_t Plan::workspace_bytes(size_t batch, bool in_place) const {
     return 0;
 }
 
+size_t Plan::workspace_used(size_t batch, bool in_place) const {
+    if (!chirp_) return workspace_bytes(batch, in_place);
+    return chirp_cols_ ? bs_m_ * 2 * real_bytes(prec_) * batch : 0;
+}
+
 void Plan::execute(const void *in, size_t in_dist, void *out, size_t out_dist, size_t batch,
                    int inverse, hipStream_t stream, void *ws, size_t ws_bytes) const {
     if (batch == 0) return;
@@ -1057,8 +1115,8 @@ void Plan::execute(const void *in, size_t in_dist, void *out, size_t out_dist, s
         const uintptr_t w0 = (uintptr_t)ws;
         if ((w0 < i0 + in_len && i0 < w0 + need) || (w0 < o0 + out_len && o0 < w0 + need))
             throw Error(SFFT_ERR_ALIASING, "workspace overlaps the input or the output");
-    } else if (need && !chirp_) {
-        if (hipMallocAsync(&owned.p, need, stream) != hipSuccess) {
+    } else if (const size_t use = workspace_used(batch, in_place)) {
+        if (hipMallocAsync(&owned.p, use, stream) != hipSuccess) {
             (void)hipGetLastError();
             owned.p = nullptr;
             throw Error(SFFT_ERR_OUT_OF_MEMORY, "workspace allocation failed");

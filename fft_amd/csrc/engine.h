@@ -100,17 +100,19 @@ class Plan {
     bool in_place_direct() const { return bs_inner_ != nullptr || passes_.size() == 1; }
     // Device workspace to hand to an execute call of `batch` transforms:
     // chirp-z rows (2 M values per transform, M the smallest 2^a 3^b 5^c
-    // convolution length; lengths that run in one launch leave it untouched)
-    // or, in place on a two-pass length, the intermediate (cn values per
+    // convolution length; plans of one launch use none of it, plans of three
+    // about half) or, in place on a two-pass length, the intermediate (cn values per
     // transform); 0 if none.
     size_t workspace_bytes(size_t batch, bool in_place) const;
+    // What such a call uses of it.
+    size_t workspace_used(size_t batch, bool in_place) const;
     // Chirp-z plan: the length has a prime factor the kernels do not plan;
     // the transform runs as a convolution through FFTs of length bluestein_m().
     bool bluestein() const { return bs_inner_ != nullptr; }
     size_t bluestein_m() const { return bs_m_; }
     const Plan *bluestein_inner() const { return bs_inner_.get(); }
     // ... in one launch, which needs no workspace (chirp.h)
-    bool bluestein_fused() const { return chirp_ != nullptr; }
+    bool bluestein_fused() const { return chirp_ && !chirp_cols_; }
 
     // in/out: device pointers; dists in elements of the in/out type
     // (complex for C2C, real/complex for the real kinds).  ws / ws_bytes: a
@@ -153,7 +155,7 @@ class Plan {
     void build_bluestein();
     template <typename T>
     void run_chirp(const void *in, int64_t din, void *out, int64_t dout, size_t batch,
-                   int inverse, hipStream_t stream) const;
+                   int inverse, hipStream_t stream, void *ws) const;
     template <typename T>
     void run_bluestein(const void *in, int64_t din, void *out, int64_t dout, size_t batch,
                        int inverse, hipStream_t stream, void *ws) const;
@@ -175,8 +177,13 @@ class Plan {
     std::unique_ptr<Plan> bs_inner_;
     size_t bs_m_ = 0;
     size_t bs_row_ = 0;  // values per workspace row of the launch sequence
-    const ChirpKernel *chirp_ = nullptr;  // the one-launch kernel, if any
-    size_t chirp_twb_ = 0;                // its second FFT's twiddles in d_tw_
+    // the one-launch kernel, or the row kernel of a plan of three launches
+    // (then with the column kernels); null: the launch sequence
+    const ChirpKernel *chirp_ = nullptr;
+    const ChirpKernel *chirp_cols_ = nullptr;
+    size_t chirp_twb_ = 0;  // second FFT's twiddles in d_tw_
+    size_t chirp_twc_ = 0;  // column kernels' twiddles
+    void *d_twist_ = nullptr;  // W_M^{k1 n2} at k1 N2 + n2 (three launches)
     void *d_chirp_ = nullptr;
     void *d_bhat_ = nullptr;
 };

@@ -52,8 +52,29 @@ const ChirpKernel *find_chirp(size_t n, int prec) {
     std::lock_guard<std::mutex> lock(registry_mutex());
     const ChirpKernel *best = nullptr;
     for (const auto &k : chirp_registry())
-        if (k.prec == prec && (size_t)k.m + 1 >= 2 * n && (!best || k.m < best->m)) best = &k;
+        if (k.part == kChirpWhole && k.prec == prec && (size_t)k.m + 1 >= 2 * n &&
+            (!best || k.m < best->m))
+            best = &k;
     return best;
+}
+
+bool find_chirp_split(size_t n, int prec, const ChirpKernel *&cols, const ChirpKernel *&rows) {
+    std::lock_guard<std::mutex> lock(registry_mutex());
+    size_t best = 0;
+    cols = rows = nullptr;
+    for (const auto &c : chirp_registry()) {
+        if (c.part != kChirpCols || c.prec != prec) continue;
+        for (const auto &r : chirp_registry()) {
+            if (r.part != kChirpRows || r.prec != prec || r.m % c.tpw) continue;
+            const size_t m = (size_t)c.m * (size_t)r.m;
+            if (m + 1 < 2 * n) continue;
+            if (best && (m > best || (m == best && c.m < cols->m))) continue;
+            best = m;
+            cols = &c;
+            rows = &r;
+        }
+    }
+    return best != 0;
 }
 
 }  // namespace sfft

@@ -74,6 +74,10 @@ template <typename T>
 hipError_t bs_gen_chirp(C2<T> *w, C2<T> *b, size_t n_len, size_t m_len, hipStream_t stream);
 template <typename T>
 hipError_t bs_scale(C2<T> *z, size_t m_len, double s, hipStream_t stream);
+// dst[k1][k2] = src[k1 + n1 k2] over m_len values
+template <typename T>
+hipError_t bs_digit_swap(const C2<T> *src, C2<T> *dst, size_t n1, size_t m_len,
+                         hipStream_t stream);
 template <typename T>
 hipError_t bs_pre(const C2<T> *in, int64_t in_dist, C2<T> *a, size_t m_len, size_t n_len,
                   size_t batch, const C2<T> *w, int mode, int conj_in, int half_shift,

@@ -1,6 +1,8 @@
-"""Chirp-z transforms that run in one launch: the smallest and the largest
-length of every compiled convolution length, all kinds and both directions,
-batches that leave part of a block idle, strided and in place.
+"""Chirp-z transforms that run in one launch or three: the smallest and the
+largest length of every compiled convolution length (three launches: of every
+column length, at the shortest and at longer rows, and the ends of the range),
+all kinds and both directions, batches that leave part of a block idle, strided
+and in place.
 
 Expected values: the DFT in 64 bits (numpy).  Tolerances are those of every
 length: rel L2 1e-6 in FP32, and in FP64 1e-13 for the complex kind; the real
@@ -18,8 +20,8 @@ from oracle import pyoracle as po
 
 pytestmark = pytest.mark.gpu
 
-M32 = [64, 128, 192, 256, 320, 384, 448, 512, 640, 768, 1024, 1280, 1536, 1792, 2048, 2560, 3072,
-       3840, 4096, 5120, 6144, 7168, 8192, 9216, 10240, 12288, 15360, 16384]
+M32 = [64, 128, 192, 256, 320, 384, 448, 512, 640, 768, 1024, 1536, 2048, 3072, 4096, 5120, 6144,
+       8192, 9216, 10240, 16384]
 M64 = [64, 128, 192, 256, 320, 384, 512, 640, 768, 1024, 1280, 1536, 2048, 2560, 3072, 3840, 4096,
        5120, 6144, 8192]
 
@@ -41,6 +43,16 @@ def _edges(ms):
     return out
 
 
+N1 = [128, 144, 160, 176, 192, 208, 240]
+# (M, n) of plans of three launches: the largest chirp-z n of N1 x 128 and of
+# N1 x 1024 (F64: 64 and 512), the first one past one launch, and the ends
+S32 = _edges([16384] + [c * 128 for c in N1[1:]])[2:] + \
+    [(c * 1024, _edges([c * 1024])[-1][1]) for c in N1[::2]] + \
+    [(240 << 14, 1966080 - 1)]
+S64 = _edges([8192] + [c * 64 for c in N1[1:]])[2:] + \
+    [(c * 512, _edges([c * 512])[-1][1]) for c in N1[1::2]] + [(240 << 13, 983040 - 1)]
+
+
 def _stream():
     return torch.cuda.current_stream().cuda_stream
 
@@ -54,8 +66,8 @@ def _spectrum(x, n, shifted):
     return out
 
 
-@pytest.mark.parametrize("prec,m,n", [(L.F32, m, n) for m, n in _edges(M32)] +
-                         [(L.F64, m, n) for m, n in _edges(M64)])
+@pytest.mark.parametrize("prec,m,n", [(L.F32, m, n) for m, n in _edges(M32) + S32] +
+                         [(L.F64, m, n) for m, n in _edges(M64) + S64])
 def test_edges_of_each_convolution_length(prec, m, n):
     cdt = np.complex64 if prec == L.F32 else np.complex128
     rdt = np.float32 if prec == L.F32 else np.float64
@@ -97,7 +109,19 @@ def test_edges_of_each_convolution_length(prec, m, n):
         assert po.rel_l2(back[0].cpu().numpy(), b64[0].cpu().numpy()) <= tol_real
 
 
-@pytest.mark.parametrize("n", [17, 1009, 8191])
+def test_launch_sequence_past_three_launches():
+    """The first length whose convolution has no compiled split."""
+    n = 1966080 + 1
+    plan = fft_amd.Plan(n, L.C2C, L.F32)
+    assert plan.info()["chirp_length"] > 240 << 14
+    x = synth.complex_uniform(n, (1, n), np.complex64)
+    xd = torch.from_numpy(x).cuda()
+    yd = torch.empty_like(xd)
+    plan.execute_ptr(xd.data_ptr(), yd.data_ptr(), 1, 0, _stream())
+    assert po.rel_l2(yd.cpu().numpy(), np.fft.fft(x.astype(np.complex128))) <= 1e-6
+
+
+@pytest.mark.parametrize("n", [17, 1009, 8191, 50021])
 def test_strided_and_workspace_rules(n):
     """Explicit distances leave the gaps alone, and the workspace a caller is
     asked for is still 2 rows of the smallest 2^a 3^b 5^c length >= 2 n - 1."""
