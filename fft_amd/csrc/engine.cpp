@@ -374,7 +374,7 @@ static bool layout_columns(int n, int prec, int max_cols, const PlanHints *h, Pa
 // kModeColRow, second kModeColCol): the pass takes its radices, threads per
 // column and columns per block, so the runtime-planned kernel (used by uneven
 // batches and strided calls) computes the same bits.
-static void use_fixed_columns(PassPlan &pp, size_t n, int prec, int mode) {
+static void use_fixed_columns(PassPlan &pp, size_t n, int prec, int mode, bool real) {
     const FixedKernel *fk = find_fixed((int)n, prec, 2, -1);
     if (!fk) return;
     // FP64 compiled columns measured faster than the runtime-planned pass
@@ -397,6 +397,20 @@ static void use_fixed_columns(PassPlan &pp, size_t n, int prec, int mode) {
     pp.lds_bytes = slot_lds * (size_t)fk->tpw;
     pp.fixed = fk;
     pp.fixed_grid[mode] = (unsigned)(fk->blocks_per_cu(mode) * device_info().cu_count);
+    if (real && fk->paired) {
+        const int pm = mode == kModeColRow ? kModeColRowPre : kModeColColPost;
+        pp.fixed_grid[pm] = (unsigned)(fk->blocks_per_cu(pm) * device_info().cu_count);
+    }
+}
+
+// A wider tile with the radices the pass has taken (so the same bits).
+static void use_wide_columns(PassPlan &pp, size_t n, int prec, int mode) {
+    const FixedKernel *fk = find_fixed((int)n, prec, 3, -1);
+    if (!fk || fk->nst != pp.pd.nstages) return;
+    for (int s = 0; s < fk->nst; ++s)
+        if (fk->radices[s] != pp.pd.st[s].radix) return;
+    pp.wide = fk;
+    pp.wide_grid = (unsigned)(fk->blocks_per_cu(mode) * device_info().cu_count);
 }
 
 // 16-bit storage: run the pass' radix-16 stages on MFMA when every wave of
@@ -580,8 +594,10 @@ Plan::Plan(size_t n, int kind, int prec, const PlanHints *h) : n_(n), kind_(kind
         // column pass for the direction (see run)
         // (16-bit plans asking for MFMA stages keep the runtime-planned pass)
         if (!(h && (h->tpw || h->fixed_variant == -2 || (stored_16(prec) && h->mfma == 1)))) {
-            use_fixed_columns(p1, n1, prec, kModeColRow);
-            use_fixed_columns(p2, n2, prec, kModeColCol);
+            use_fixed_columns(p1, n1, prec, kModeColRow, kind != kC2C);
+            use_fixed_columns(p2, n2, prec, kModeColCol, kind != kC2C);
+            use_wide_columns(p1, n1, prec, kModeColRow);
+            use_wide_columns(p2, n2, prec, kModeColCol);
         }
         passes_.push_back(p1);
         passes_.push_back(p2);
@@ -924,6 +940,8 @@ void Plan::run(const void *in, size_t in_dist, void *out, size_t out_dist, size_
     run_passes<T>(in, din, out, dout, batch, inverse, stream, ws);
 }
 
+static int plain_column_mode(size_t p) { return p == 0 ? kModeColRow : kModeColCol; }
+
 // The passes of a direct plan over one batch (distances in complex values).
 template <typename T>
 void Plan::run_passes(const void *in, int64_t din, void *out, int64_t dout, size_t batch,
@@ -933,6 +951,7 @@ void Plan::run_passes(const void *in, int64_t din, void *out, int64_t dout, size
     // the workspace (cn values per transform) and the second pass reads it
     // there; out of place the output buffer holds the intermediate.
     const int64_t dws = (int64_t)cn_;
+    bool posted = false;
     for (size_t p = 0; p < np; ++p) {
         const PassPlan &pp = passes_[p];
         const bool last = p + 1 == np;
@@ -942,17 +961,19 @@ void Plan::run_passes(const void *in, int64_t din, void *out, int64_t dout, size
         const int64_t ddst = (!last && ws) ? dws : dout;
         const size_t slots = batch * (size_t)pp.slots_per_transform;
         if (slots > 0x7fffffffull) throw Error(SFFT_ERR_INVALID_ARG, "batch too large");
-        if (pp.fixed && pp.fixed->real == 2) {
-            // compiled column kernel where the pass is a plain column pass:
-            // complex passes, and real passes with no pre-process or rotation
-            // fused into their loads / stores for this direction
-            const PassArgs<T> m = pass_args<T>(p, inverse);
-            const bool plain = m.mode == kModeC2C ||
-                               ((m.mode == kModeR2CLoad || m.mode == kModeC2RStore) && !m.half_shift);
-            if (plain) {
-                run_fixed_columns<T>(p, src, dsrc, dst, ddst, batch, inverse, stream);
-                continue;
-            }
+        const int cm = column_mode(p, inverse);
+        if (cm >= 0 && cm == plain_column_mode(p) && pp.wide &&
+            pp.slots_per_transform % pp.wide->tpw == 0 &&
+            slots / (size_t)pp.wide->tpw >= (size_t)device_info().cu_count) {
+            run_fixed_columns<T>(p, *pp.wide, cm, pp.wide_grid, src, dsrc, dst, ddst, batch,
+                                 inverse, stream);
+            continue;
+        }
+        if (cm >= 0 && pp.fixed_grid[cm]) {
+            run_fixed_columns<T>(p, *pp.fixed, cm, pp.fixed_grid[cm], src, dsrc, dst, ddst, batch,
+                                 inverse, stream);
+            posted |= cm == kModeColColPost;
+            continue;
         }
         PassArgs<T> a = pass_args<T>(p, inverse);
         a.iin.batch_stride = dsrc;
@@ -977,8 +998,9 @@ void Plan::run_passes(const void *in, int64_t din, void *out, int64_t dout, size
         }
         check_hip(launch_pass<T>(a, pp.ept, grid, pp.block, pp.lds_bytes, stream), "pass launch");
     }
-    // two-pass forward real: pairwise post-process in place on the output
-    if (kind_ != kC2C && !inverse && np > 1)
+    // two-pass forward real: pairwise post-process in place on the output,
+    // where the second pass did not do it
+    if (kind_ != kC2C && !inverse && np > 1 && !posted)
         check_hip(launch_real_post<T>((C2<T> *)out, dout, (int)cn_, batch,
                                       (const C2<T> *)d_real_tw_, kind_ == kR2CHalf, stream),
                   "real post-process launch");
@@ -1016,19 +1038,41 @@ void Plan::run_fixed(const void *in, void *out, size_t batch, int inverse,
 }
 template void Plan::run_fixed<float>(const void *, void *, size_t, int, hipStream_t) const;
 
-// Pass p of a two-pass complex plan through its compiled column kernel.  The
+// Compiled column kernels run plain column passes (complex ones, and real ones
+// with no rotation at their loads or stores) and the paired passes of real
+// transforms; -1 otherwise.
+int Plan::column_mode(size_t p, int inverse) const {
+    const PassPlan &pp = passes_[p];
+    if (passes_.size() != 2) return -1;
+    const int plain = plain_column_mode(p);
+    if (kind_ == kC2C) return plain;
+    if (p == 0 ? inverse : !inverse) {  // the pass with the pairs
+        const int pm = p == 0 ? kModeColRowPre : kModeColColPost;
+        if (pp.fixed && pp.fixed_grid[pm]) return pm;
+        return p == 0 ? -1 : plain;
+    }
+    return kind_ == kR2CHalf ? -1 : plain;
+}
+
+// Pass p of a two-pass plan through its compiled column kernel.  The
 // kernel addresses HBM with 32-bit byte offsets from the launch base, so the
 // batch is split into launches spanning less than 4 GiB.
 template <typename T>
-void Plan::run_fixed_columns(size_t p, const void *src, int64_t dsrc, void *dst, int64_t ddst,
-                             size_t batch, int inverse, hipStream_t stream) const {
+void Plan::run_fixed_columns(size_t p, const FixedKernel &fk, int mode, unsigned resident,
+                             const void *src, int64_t dsrc, void *dst, int64_t ddst, size_t batch,
+                             int inverse, hipStream_t stream) const {
     const PassPlan &pp = passes_[p];
-    const FixedKernel &fk = *pp.fixed;
-    const int mode = p == 0 ? kModeColRow : kModeColCol;
+    const bool paired = mode == kModeColRowPre || mode == kModeColColPost;
+    // slots per transform: a column each, or the slots of its pair tiles
+    const uint32_t columns = (uint32_t)pp.slots_per_transform;
+    const uint32_t half = (uint32_t)fk.tpw / 2;
+    const uint32_t tiles =
+        paired ? (pair_columns(columns, kind_ == kR2CHalf) + half - 1) / half : 0;
+    const size_t slots = paired ? (size_t)tiles * (size_t)fk.tpw : columns;
     const size_t eb = 2 * real_bytes(prec_);  // bytes per complex value in HBM
     const int64_t dmax = std::max(dsrc, ddst);
     const size_t chunk = std::max<size_t>(1, ((1ull << 32) - 1) / ((size_t)dmax * eb));
-    if ((size_t)pp.slots_per_transform * std::min(chunk, batch) > 0x7fffffffull)
+    if (slots * std::min(chunk, batch) > 0x7fffffffull)
         throw Error(SFFT_ERR_INVALID_ARG, "batch too large");
     const uint32_t flip = 0x80000000u;
     const PassArgs<T> conj = pass_args<T>(p, inverse);  // the pass' conjugations
@@ -1040,10 +1084,13 @@ void Plan::run_fixed_columns(size_t p, const void *src, int64_t dsrc, void *dst,
         a.in = (const C2<T> *)((const char *)src + (int64_t)c0 * dsrc * (int64_t)eb);
         a.out = (C2<T> *)((char *)dst + (int64_t)c0 * ddst * (int64_t)eb);
         a.tw = (const C2<T> *)d_tw_ + tw0;
-        a.total_slots = (int32_t)(cb * (size_t)pp.slots_per_transform);
+        a.total_slots = (int32_t)(cb * slots);
         a.flip_in = conj.conj_in ? flip : 0u;
         a.flip_out = conj.conj_out ? flip : 0u;
-        a.spt = make_fastdiv((uint32_t)pp.slots_per_transform);
+        a.spt = make_fastdiv(columns);
+        if (paired) a.tiles = make_fastdiv(tiles);
+        a.real_tw = (const C2<T> *)d_real_tw_;
+        a.half_shift = kind_ == kR2CHalf;
         a.in_bs = (int32_t)dsrc;
         a.in_ss = (int32_t)pp.in_slot_stride;
         a.in_es = (int32_t)pp.in_elem_stride;
@@ -1056,14 +1103,16 @@ void Plan::run_fixed_columns(size_t p, const void *src, int64_t dsrc, void *dst,
         a.ptw_coarse = (const C2<T> *)d_ptw_coarse_;
         a.ptw_full = (const C2<T> *)d_ptw_full_;
         const size_t groups = ((size_t)a.total_slots + fk.tpw - 1) / fk.tpw;
-        const unsigned grid = (unsigned)std::min<size_t>(groups, pp.fixed_grid[mode]);
+        const unsigned grid = (unsigned)std::min<size_t>(groups, resident);
         check_hip(fk.launch(&a, mode, grid, stream), "column-pass launch");
     }
 }
-template void Plan::run_fixed_columns<float>(size_t, const void *, int64_t, void *, int64_t,
-                                             size_t, int, hipStream_t) const;
-template void Plan::run_fixed_columns<double>(size_t, const void *, int64_t, void *, int64_t,
-                                              size_t, int, hipStream_t) const;
+template void Plan::run_fixed_columns<float>(size_t, const FixedKernel &, int, unsigned,
+                                             const void *, int64_t, void *, int64_t, size_t, int,
+                                             hipStream_t) const;
+template void Plan::run_fixed_columns<double>(size_t, const FixedKernel &, int, unsigned,
+                                              const void *, int64_t, void *, int64_t, size_t, int,
+                                              hipStream_t) const;
 template void Plan::run_fixed<double>(const void *, void *, size_t, int, hipStream_t) const;
 
 size_t Plan::workspace_bytes(size_t batch, bool in_place) const {

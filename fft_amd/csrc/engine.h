@@ -67,7 +67,11 @@ struct PassPlan {
     size_t lds_bytes = 0;
     // compile-time planned kernel with the same radices (contiguous batches)
     const FixedKernel *fixed = nullptr;
-    unsigned fixed_grid[8] = {};  // resident blocks per mode (kModeC2C ... kModeColCol)
+    unsigned fixed_grid[kModes] = {};  // resident blocks per mode
+    // wider tiles of a plain column pass (same bits), for launches that give
+    // every CU a tile
+    const FixedKernel *wide = nullptr;
+    unsigned wide_grid = 0;
 };
 
 // Overrides the planner's choice (autotuner candidates).
@@ -146,10 +150,13 @@ class Plan {
     template <typename T>
     void run_passes(const void *in, int64_t din, void *out, int64_t dout, size_t batch,
                     int inverse, hipStream_t stream, void *ws) const;
+    // The mode in which compiled column kernels run pass p in a direction.
+    int column_mode(size_t p, int inverse) const;
     template <typename T>
     void run_fixed(const void *in, void *out, size_t batch, int inverse, hipStream_t stream) const;
     template <typename T>
-    void run_fixed_columns(size_t p, const void *src, int64_t dsrc, void *dst, int64_t ddst,
+    void run_fixed_columns(size_t p, const FixedKernel &fk, int mode, unsigned resident,
+                           const void *src, int64_t dsrc, void *dst, int64_t ddst,
                            size_t batch, int inverse, hipStream_t stream) const;
     template <typename T>
     void build_bluestein();

@@ -39,7 +39,24 @@ struct FixedArgs {
     int32_t post_tw, ptw_shift;  // first pass: output element e times W_N^{c e}
     const C2<T> *ptw_fine, *ptw_coarse;
     const C2<T> *ptw_full;  // or null: W_N^{c e} at c N + e (N: this pass' length)
+    FastDiv tiles;  // paired column modes: tiles per transform
 };
+
+// Paired column modes.  Bin m = c + S e of a two-pass real transform (column c
+// of S = spt, element e of N) pairs with h - m (h - 1 - m for the half shift),
+// h = S N: element N - 1 - e of the mirror column S - c (S - 1 - c).  Only
+// column 0 (without the shift) pairs within itself at N - e, and the middle
+// column at N - 1 - e.  A tile of TPW slots therefore holds TPW / 2 adjacent
+// columns and, in the other half of its slots, their mirror columns, and the
+// pair sums need nothing from outside the tile: the values are exchanged
+// through LDS once (forward: after the last stage; inverse: before the first).
+// Without this the forward transform ran a third pass over the output
+// (k_real_post) and the inverse the runtime-planned pass with two gathered
+// loads an element: 96000 x 512 forward 231 -> 204 us, inverse 246 -> 199;
+// 131072 x 256 158 -> 122 and 152 -> 128.
+__host__ __device__ inline uint32_t pair_columns(uint32_t s, bool shifted) {
+    return (shifted ? (s - 1) / 2 : s / 2) + 1;  // columns that are not mirror images
+}
 
 // Sign flip of the imaginary part by a uniform xor mask (0 or the sign bit).
 __device__ __forceinline__ void flip_im(C2<float> &x, uint32_t m) {
@@ -109,17 +126,21 @@ struct Fixed {
     // Column modes: stage 0 (and the last stage of the second pass) map
     // adjacent lanes to adjacent slots (columns), so the strided HBM accesses
     // coalesce across columns; the other stages keep slot-major lanes.
-    static constexpr bool COL = MODE == kModeColRow || MODE == kModeColCol;
+    static constexpr bool PRE = MODE == kModeColRowPre, POST = MODE == kModeColColPost;
+    static constexpr bool PAIR = PRE || POST;
+    static constexpr bool COL = MODE == kModeColRow || MODE == kModeColCol || PAIR;
     static constexpr bool COL_OUT = MODE == kModeColCol;
     static constexpr int PADSH = SCH::PADSH;
     static constexpr int pad(int e) { return e + (e >> PADSH); }
     static constexpr int STRIDE = N + (N >> PADSH) + 1;
     static constexpr uint32_t EB = sizeof(C2<T>);  // bytes per element in LDS
-    static constexpr uint32_t DB =                  // and in HBM
-        ST::native ? sizeof(C2<T>) : 2 * sizeof(uint16_t);
+    static constexpr uint32_t DB = ST::kBytes;      // and in HBM
     static constexpr bool NT_MODE = MODE != kModeC2R || (SCH::NT & 4);
-    static constexpr bool NT_LD = ST::native && (SCH::NT & 1) && NT_MODE && MODE != kModeColCol;
-    static constexpr bool NT_ST = ST::native && (SCH::NT & 2) && NT_MODE && MODE != kModeColRow;
+    // (the mirror columns of neighbouring pair tiles share lines: no hint)
+    static constexpr bool NT_LD =
+        ST::native && (SCH::NT & 1) && NT_MODE && MODE != kModeColCol && !PAIR;
+    static constexpr bool NT_ST =
+        ST::native && (SCH::NT & 2) && NT_MODE && MODE != kModeColRow && !PAIR;
     using V2 = T __attribute__((ext_vector_type(2)));
     static __device__ __forceinline__ C2<T> ld(const char *p) {
         if constexpr (NT_LD) {
@@ -158,11 +179,54 @@ struct Fixed {
     // The next group's first-stage loads are issued in stage PF_STAGE, after
     // the twiddle loads of that stage and of the next one: vector-memory
     // counters drain in issue order, so waiting for a twiddle never waits for
-    // the (slower) HBM prefetch.
+    // the (slower) HBM prefetch.  (The inverse paired mode issues them a stage
+    // later: with the pairs' values they need too many registers in stage 0,
+    // 180 -> 145 us at 100000 x 160; with a first radix of 25 that measured
+    // the other way round, 211 -> 230 us at 46875 x 400.)
     static constexpr int PF_STAGE =
-        PFS >= 0 ? (PFS < NST ? PFS : NST - 1) : ((NST + PFS) > 0 ? (NST + PFS) : 0);
+        PRE && RAD[0] <= 16 ? 1 : PFS >= 0 ? (PFS < NST ? PFS : NST - 1) : ((NST + PFS) > 0 ? (NST + PFS) : 0);
     static_assert(ns_of(NST) == N, "radices must multiply to N");
     static_assert(!COL || NST >= 2, "column kernels need two stages or more");
+
+    // Column c of transform t in slot `slot` of the pass' slot g (g = first
+    // slot of the group + slot); false if the slot holds none.
+    static __device__ __forceinline__ bool column_of(const FixedArgs<T> &a, int g, uint32_t &t,
+                                                     uint32_t &c) {
+        if constexpr (PAIR) {
+            const uint32_t q = (uint32_t)g / TPW, slot = (uint32_t)g % TPW;
+            const uint32_t s = a.spt.d;
+            const bool mod = a.half_shift != 0;
+            t = fdiv(q, a.tiles);
+            const uint32_t cp = (q - t * a.tiles.d) * (TPW / 2) + slot % (TPW / 2);
+            c = cp;
+            if (g >= a.total_slots || cp >= pair_columns(s, mod)) return false;
+            if (slot < TPW / 2) return true;
+            c = mod ? s - 1 - cp : s - cp;
+            return c != cp && c < s;  // (a column that pairs within itself has no mirror)
+        } else {
+            t = fdiv((uint32_t)g, a.spt);
+            c = (uint32_t)g - t * a.spt.d;
+            return g < a.total_slots;
+        }
+    }
+
+    // Partner of element e of the column c in slot `slot`: LDS index.
+    static __device__ __forceinline__ int partner(const FixedArgs<T> &a, uint32_t c, int slot,
+                                                  int e) {
+        const uint32_t s = a.spt.d;
+        const bool mod = a.half_shift != 0;
+        const bool own = mod ? 2 * c + 1 == s : (c == 0 || 2 * c == s);
+        const int ps = own ? slot : (slot + TPW / 2) % TPW;
+        const int pe = (!mod && c == 0) ? (e == 0 ? 0 : N - e) : N - 1 - e;
+        return ps * STRIDE + pad(pe);
+    }
+    // Pair index i of bin m (whose table entry both of its bins use): the
+    // smaller of the two, but h / 2 for the shifted kind's middle pair.
+    static __device__ __forceinline__ uint32_t pair_index(uint32_t m, uint32_t h, bool mod) {
+        const uint32_t mm = mod ? h - 1 - m : h - m;
+        const uint32_t i = m < mm ? m : mm;
+        return (mod && (h & 1) == 0 && i == h / 2 - 1) ? h / 2 : i;
+    }
 
     // thread -> (slot, element lane) of stage S; gbase = first slot of the group
     template <int S>
@@ -225,8 +289,8 @@ struct Fixed {
         if (g >= a.total_slots) return;
         const char *src = reinterpret_cast<const char *>(a.in);
         if constexpr (COL) {
-            const uint32_t t = fdiv((uint32_t)g, a.spt);
-            const uint32_t c = (uint32_t)g - t * a.spt.d;
+            uint32_t t, c;
+            if (!column_of(a, g, t, c) && PAIR) return;
             const uint32_t es = (uint32_t)a.in_es * DB;
             const uint32_t lane =
                 (t * (uint32_t)a.in_bs + c * (uint32_t)a.in_ss) * DB + (uint32_t)lid * es;
@@ -272,7 +336,7 @@ struct Fixed {
             map_of<0>(a, g_in, gx, sx, lid_pf, ax);
         }
         constexpr bool FIRST = (S == 0), LAST = (S == NST - 1);
-        constexpr bool SRC_PF = FIRST && MODE != kModeC2R;
+        constexpr bool SRC_PF = FIRST && MODE != kModeC2R && !PRE;
         constexpr bool DST_G = LAST && MODE != kModeR2C;
         constexpr bool SEP_R = ct_pow2(NB) || (NB % (1 << PADSH)) == 0;
         constexpr bool SEP_W = (NS % (1 << PADSH)) == 0 || (ct_pow2(NS) && ct_pow2(R));
@@ -290,6 +354,22 @@ struct Fixed {
                     flip_im(v[b][r], a.flip_in);
                 }
         }
+        // inverse real: the raw bins of the tile to LDS, their pairs'
+        // pre-process there (its table loads go before the prefetch, as every
+        // other table load)
+        constexpr bool PRE_HERE = FIRST && PRE;
+        PairWork<PRE_HERE> pair;
+        if constexpr (PRE_HERE) {
+            C2<T> *ls = reinterpret_cast<C2<T> *>(lds_c);
+#pragma unroll
+            for (int b = 0; b < B; ++b)
+                if (jvalid(b)) {
+#pragma unroll
+                    for (int r = 0; r < R; ++r)
+                        ls[slot * STRIDE + pad(lid + b * TPT + r * NB)] = pf[b * R + r];
+                }
+            pair.init(a, g - slot);
+        }
         if constexpr (!TW_READY) load_tw<S>(a, tb, active, lid);
         if constexpr (PF_HERE) {
             if constexpr (SCH::PF_FIRST) {
@@ -299,6 +379,11 @@ struct Fixed {
                 load_tw<S + 1>(a, tn, active_n, lid_n);
                 if (MODE != kModeC2R && g_next >= 0) load0(a, pf, g_next, lid_pf);
             }
+        }
+        if constexpr (PRE_HERE) {
+            __syncthreads();
+            pair_pre(a, reinterpret_cast<C2<T> *>(lds_c), pair);
+            __syncthreads();
         }
         if constexpr (SRC_PF) {
             if (MODE == kModeR2C && a.half_shift) {
@@ -342,10 +427,29 @@ struct Fixed {
                 dft<R, T>(v[b]);
             }
         }
-        if constexpr (DST_G && COL) {
+        if constexpr (DST_G && POST) {
+            // the spectrum's tile to LDS, then its pairs to HBM
+            // (signalsmith-fft.h:459-472)
+            C2<T> *ls = reinterpret_cast<C2<T> *>(lds_c);
+#pragma unroll
+            for (int b = 0; b < B; ++b) {
+                const int j = lid + b * TPT;
+                if (jvalid(b)) {
+#pragma unroll
+                    for (int t2 = 0; t2 < R; ++t2)
+                        ls[slot * STRIDE + pad((j / NS) * NS * R + j % NS + t2 * NS)] = v[b][t2];
+                }
+            }
+            PairWork<true> pair_out;
+            pair_out.init(a, g - slot);
+            __syncthreads();
+            pair_post(a, ls, pair_out);
+            __syncthreads();  // the tile is read before the next one's exchange
+        } else if constexpr (DST_G && COL) {
             char *dst = reinterpret_cast<char *>(a.out);
-            const uint32_t t = fdiv((uint32_t)g, a.spt);
-            const uint32_t c = (uint32_t)g - t * a.spt.d;
+            uint32_t t, c;
+            const bool held = column_of(a, g, t, c);
+            if constexpr (PAIR) active = held;
             const uint32_t es = (uint32_t)a.out_es * DB;
             const uint32_t sbase = (t * (uint32_t)a.out_bs + c * (uint32_t)a.out_ss) * DB;
             const uint32_t mask = (1u << a.ptw_shift) - 1u;
@@ -431,6 +535,97 @@ struct Fixed {
             }
             __syncthreads();
         }
+    }
+
+    // A thread's pairs of a paired tile: column c in its slot (of the first
+    // TPW / 2), elements e0 + k STEP, and their table entries.
+    template <bool USED>
+    struct PairWork {};
+    template <>
+    struct PairWork<true> {
+        static constexpr int H = TPW > 1 ? TPW / 2 : 1, STEP = THREADS / H,
+                             IT = (N + STEP - 1) / STEP;
+        int slot, e0;
+        uint32_t t, c;
+        bool held;
+        C2<T> w[IT];
+        __device__ __forceinline__ void init(const FixedArgs<T> &a, int gbase) {
+            slot = (int)threadIdx.x % H;
+            e0 = (int)threadIdx.x / H;
+            held = column_of(a, gbase + slot, t, c) && e0 < STEP;
+            const uint32_t s = a.spt.d, h = s * (uint32_t)N;
+#pragma unroll
+            for (int k = 0; k < IT; ++k) {
+                const int e = e0 + k * STEP;
+                w[k] = a.real_tw[held && e < N
+                                     ? pair_index(c + s * (uint32_t)e, h, a.half_shift != 0)
+                                     : 0u];
+            }
+        }
+        // Calls f(k, z, o, m, mm, first): bins m (LDS place z) and mm (place
+        // o) of each pair; first: m is the pair's bin i.
+        template <typename F>
+        __device__ __forceinline__ void each(const FixedArgs<T> &a, F &&f) const {
+            if (!held) return;
+            const uint32_t s = a.spt.d, h = s * (uint32_t)N;
+            const bool mod = a.half_shift != 0;
+            // within one column each pair is met from both sides
+            const bool own = mod ? 2 * c + 1 == s : (c == 0 || 2 * c == s);
+#pragma unroll
+            for (int k = 0; k < IT; ++k) {
+                const int e = e0 + k * STEP;
+                if (e >= N) continue;
+                const uint32_t m = c + s * (uint32_t)e;
+                const uint32_t mm = mod ? h - 1 - m : h - m;
+                if (own && m > mm && m != 0) continue;
+                f(k, slot * STRIDE + pad(e), partner(a, c, slot, e), m, mm,
+                  pair_index(m, h, mod) == m);
+            }
+        }
+    };
+
+    // Forward real post-process of a tile whose spectrum is in LDS: both bins
+    // of each pair stored at base + bin (rows of TPW / 2 columns).
+    static __device__ __forceinline__ void pair_post(const FixedArgs<T> &a, const C2<T> *ls,
+                                                     const PairWork<true> &p) {
+        const bool mod = a.half_shift != 0;
+        char *dst = reinterpret_cast<char *>(a.out) + (size_t)(p.t * (uint32_t)a.out_bs) * DB;
+        const T half = (T)0.5;
+        p.each(a, [&](int k, int z, int o, uint32_t m, uint32_t mm, bool first) {
+            const C2<T> zm = ls[z], zo = ls[o];
+            if (!mod && m == 0) {
+                st(dst, {zm.x + zm.y, zm.x - zm.y});
+                return;
+            }
+            const uint32_t i = first ? m : mm, ci = first ? mm : m;
+            const C2<T> zi = first ? zm : zo, zc = first ? zo : zm;
+            const C2<T> odd = {(zi.x + zc.x) * half, (zi.y - zc.y) * half};
+            const C2<T> ev = {(zi.x - zc.x) * half, (zi.y + zc.y) * half};
+            const C2<T> ew = cmul(ev, p.w[k]);
+            if (i != ci) st(dst + i * DB, cadd(odd, ew));
+            st(dst + ci * DB, cconj(csub(odd, ew)));
+        });
+    }
+
+    // Inverse real pre-process of a tile's raw bins in LDS, in place: conj(.)
+    // of each pre-processed bin (signalsmith-fft.h:478-492).
+    static __device__ __forceinline__ void pair_pre(const FixedArgs<T> &a, C2<T> *ls,
+                                                    const PairWork<true> &p) {
+        const bool mod = a.half_shift != 0;
+        p.each(a, [&](int k, int z, int o, uint32_t m, uint32_t mm, bool first) {
+            const C2<T> xm = ls[z], xo = ls[o];
+            if (!mod && m == 0) {
+                ls[z] = {xm.x + xm.y, -(xm.x - xm.y)};
+                return;
+            }
+            const int li = first ? z : o, lc = first ? o : z;
+            const C2<T> x = first ? xm : xo, x2 = first ? xo : xm;
+            const C2<T> odd = {x.x + x2.x, x.y - x2.y};
+            const C2<T> erot = {x.x - x2.x, x.y + x2.y};
+            const C2<T> ev = cmulc(erot, p.w[k]);
+            if (li != lc) ls[li] = cconj(cadd(odd, ev));
+            ls[lc] = csub(odd, ev);  // conj(conj(odd - ev))
+        });
     }
 
     template <int S, bool TW_READY>
@@ -540,7 +735,7 @@ struct Fixed {
             const auto odd_pitch = [](int32_t es) {
                 return es != 1 && (((uint32_t)es * DB) & 127u) != 0;
             };
-            const bool share = NARROW || odd_pitch(a.in_es) || odd_pitch(a.out_es);
+            const bool share = PAIR || NARROW || odd_pitch(a.in_es) || odd_pitch(a.out_es);
             const int off = share ? (int)xcd_tile(blockIdx.x, (unsigned)G) : (int)blockIdx.x;
             int grp = off;
             if (grp < ngroups) load0(a, pf, grp * TPW + slot0, lid0);
@@ -584,6 +779,8 @@ struct FixedKernel {
     int prec;       // 0 F32, 1 F64
     int real;       // 0: C2C kernel; 1: real pair (R2C forward + C2R inverse);
                     // 2: column passes of two-pass plans (kModeColRow, kModeColCol)
+                    // 3: the same in wider tiles, for launches that fill the device
+    bool paired;    // 2: with the paired modes of real transforms
     int tpt, tpw;
     int nst;
     int radices[kMaxStages];
@@ -676,32 +873,51 @@ struct FixedReal {
     }
 };
 
-// Registers the column-pass pair of one compile-time plan of column length
-// N (registry kind 2): the first pass of a two-pass plan (kModeColRow) and
-// the second (kModeColCol).
-template <typename T, int N, int TPT, int TPW, class SCH, int VARIANT, int... Rs>
-struct FixedCol {
-    using F1 = Fixed<T, N, TPT, TPW, kModeColRow, SCH, Rs...>;
-    using F2 = Fixed<T, N, TPT, TPW, kModeColCol, SCH, Rs...>;
-    FixedCol() {
+// Registers the column passes of one compile-time plan of column length N
+// (registry kind 2): the first pass of a two-pass plan (kModeColRow), the
+// second (kModeColCol), and with REAL their paired forms for real transforms
+// (kModeColRowPre, kModeColColPost).  KIND 3: a wider tile of the same radices.
+template <typename T, int N, int TPT, int TPW, class SCH, int VARIANT, bool REAL, int KIND,
+          int... Rs>
+struct FixedColOf {
+    template <int MODE>
+    using F = Fixed<T, N, TPT, TPW, MODE, SCH, Rs...>;
+    FixedColOf() {
         FixedKernel k{};
         k.n = N;
         k.variant = VARIANT;
         k.prec = FixedElem<T>::prec;
-        k.real = 2;
+        k.real = KIND;
+        k.paired = REAL;
         k.tpt = TPT;
         k.tpw = TPW;
         fixed_fill_radices<Rs...>(k);
-        k.lds_bytes = F1::LDS_BYTES;
+        k.lds_bytes = F<kModeColRow>::LDS_BYTES;
         k.launch = [](const void *args, int mode, unsigned grid, hipStream_t s) {
-            return mode == kModeColCol ? fixed_launch_one<F2>(args, grid, s)
-                                       : fixed_launch_one<F1>(args, grid, s);
+            if constexpr (REAL) {
+                if (mode == kModeColRowPre)
+                    return fixed_launch_one<F<kModeColRowPre>>(args, grid, s);
+                if (mode == kModeColColPost)
+                    return fixed_launch_one<F<kModeColColPost>>(args, grid, s);
+            }
+            return mode == kModeColCol ? fixed_launch_one<F<kModeColCol>>(args, grid, s)
+                                       : fixed_launch_one<F<kModeColRow>>(args, grid, s);
         };
         k.blocks_per_cu = [](int mode) {
-            return mode == kModeColCol ? fixed_occupancy<F2>() : fixed_occupancy<F1>();
+            if constexpr (REAL) {
+                if (mode == kModeColRowPre) return fixed_occupancy<F<kModeColRowPre>>();
+                if (mode == kModeColColPost) return fixed_occupancy<F<kModeColColPost>>();
+            }
+            return mode == kModeColCol ? fixed_occupancy<F<kModeColCol>>()
+                                       : fixed_occupancy<F<kModeColRow>>();
         };
         register_fixed(k);
     }
 };
+template <typename T, int N, int TPT, int TPW, class SCH, int VARIANT, int... Rs>
+using FixedCol =
+    FixedColOf<T, N, TPT, TPW, SCH, VARIANT, std::is_arithmetic<T>::value, 2, Rs...>;
+template <typename T, int N, int TPT, int TPW, class SCH, int VARIANT, int... Rs>
+using FixedColWide = FixedColOf<T, N, TPT, TPW, SCH, VARIANT, false, 3, Rs...>;
 
 }  // namespace sfft

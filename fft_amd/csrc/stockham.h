@@ -62,7 +62,12 @@ enum : int32_t {
     // compiled column-pass kernels of two-pass plans (fixed.h only)
     kModeColRow = 6,  // first pass: column loads, four-step twiddle, row stores
     kModeColCol = 7,  // second pass: column loads and column stores
+    // the same with the pairs (i, h - i) of two-pass real transforms fused in;
+    // a tile holds columns and their mirror images
+    kModeColRowPre = 8,   // first pass, inverse: pre-process at the column loads
+    kModeColColPost = 9,  // second pass, forward: post-process at the column stores
 };
+constexpr int kModes = 10;
 
 // The pair loops of the real pre-/post-process (signalsmith-fft.h:463-472,
 // :482-492) visit i = 0..h/2 (1..h/2 without the half shift) with partner
