@@ -940,6 +940,11 @@ void Plan::run(const void *in, size_t in_dist, void *out, size_t out_dist, size_
     run_passes<T>(in, din, out, dout, batch, inverse, stream, ws);
 }
 
+// Columns per block of a column kernel in a mode.
+static int column_tile(const FixedKernel &fk, int mode) {
+    return mode == kModeColRow ? fk.row_tpw : mode == kModeColCol ? fk.col_tpw : fk.tpw;
+}
+
 static int plain_column_mode(size_t p) { return p == 0 ? kModeColRow : kModeColCol; }
 
 // The passes of a direct plan over one batch (distances in complex values).
@@ -1063,12 +1068,13 @@ void Plan::run_fixed_columns(size_t p, const FixedKernel &fk, int mode, unsigned
                              int inverse, hipStream_t stream) const {
     const PassPlan &pp = passes_[p];
     const bool paired = mode == kModeColRowPre || mode == kModeColColPost;
+    const int tpw = column_tile(fk, mode);
     // slots per transform: a column each, or the slots of its pair tiles
     const uint32_t columns = (uint32_t)pp.slots_per_transform;
-    const uint32_t half = (uint32_t)fk.tpw / 2;
+    const uint32_t half = (uint32_t)tpw / 2;
     const uint32_t tiles =
         paired ? (pair_columns(columns, kind_ == kR2CHalf) + half - 1) / half : 0;
-    const size_t slots = paired ? (size_t)tiles * (size_t)fk.tpw : columns;
+    const size_t slots = paired ? (size_t)tiles * (size_t)tpw : columns;
     const size_t eb = 2 * real_bytes(prec_);  // bytes per complex value in HBM
     const int64_t dmax = std::max(dsrc, ddst);
     const size_t chunk = std::max<size_t>(1, ((1ull << 32) - 1) / ((size_t)dmax * eb));
@@ -1102,7 +1108,7 @@ void Plan::run_fixed_columns(size_t p, const FixedKernel &fk, int mode, unsigned
         a.ptw_fine = (const C2<T> *)d_ptw_fine_;
         a.ptw_coarse = (const C2<T> *)d_ptw_coarse_;
         a.ptw_full = (const C2<T> *)d_ptw_full_;
-        const size_t groups = ((size_t)a.total_slots + fk.tpw - 1) / fk.tpw;
+        const size_t groups = ((size_t)a.total_slots + tpw - 1) / tpw;
         const unsigned grid = (unsigned)std::min<size_t>(groups, resident);
         check_hip(fk.launch(&a, mode, grid, stream), "column-pass launch");
     }

@@ -7,10 +7,22 @@
 // (same butterflies, same twiddle table, explicit FMAs), so a plan gives the
 // same bits on either path.
 //
-// Persistent + pipelined: a block walks slot groups blockIdx.x,
-// blockIdx.x + gridDim.x, ...; the first stage of a group takes its elements
-// from registers loaded during the previous group, and right after that the
-// next group's loads are issued, so HBM reads overlap the remaining stages.
+// Two schedules:
+//  - One group of slots per block.  Several blocks share a CU, and one's loads
+//    overlap another's stages.  With nothing carried round a loop the kernels
+//    need 54-90 registers in FP32 instead of 100-170 (the compiler hoists
+//    every stage's addresses out of a persistent loop), so 16 to 32 waves stay
+//    resident.
+//  - Persistent + pipelined, where the tile leaves room for one block per CU
+//    only: a block walks groups blockIdx.x, blockIdx.x + gridDim.x, ...; the
+//    first stage of a group takes its elements from registers loaded during
+//    the previous group, and right after that the next group's loads are
+//    issued, so HBM reads overlap the remaining stages.
+// The first measured faster at nearly every length whose tile is 80 KB or
+// less (256 MB launches, first / second): complex FP32 median 1.08x of 106
+// lengths, FP64 1.05x of 112 up to 4860, real 1.13x forward and 1.17x inverse
+// of 98 (up to 2.0x), column passes 1.09x (first pass) and 1.19x (second) of
+// 38; the second at nearly every length above it (0.80-0.96x).
 #pragma once
 
 #include "stockham.h"
@@ -86,6 +98,11 @@ __device__ __forceinline__ void flip_im(C2<double> &x, uint32_t m) {
 //         the forward kernel made it 10 % faster and the inverse leg that
 //         follows it 10 % slower, with no net gain; they are not used there.)
 constexpr int kLdsNoPad = 30;
+constexpr int kNoPrefetch = -100;  // PFS: never persistent
+constexpr int kPersist = 100;      // PFS + kPersist: persistent at any tile size
+constexpr unsigned kXcdWindow = 256;  // blocks numbered XCD-contiguously together
+// Largest tile of which two blocks fit a CU.
+constexpr size_t kSharedCuLds = 80 * 1024;
 template <int PFS_, int MINW_, int PAIR_ = 1, int PF_FIRST_ = 0, int PADSH_ = kLdsPadShift,
           int NT_ = 0>
 struct Sched {
@@ -107,6 +124,12 @@ struct FixedElem {
     using S = StoreNative;
     static constexpr int prec = sizeof(E) == 8 ? 1 : 0;
 };
+template <>
+struct FixedElem<Stored<StoreF32>> {  // FP32 in HBM under FP64 arithmetic
+    using T = double;
+    using S = StoreF32;
+    static constexpr int prec = 4;
+};
 template <class S_>
 struct FixedElem<Stored<S_>> {
     using T = float;
@@ -118,7 +141,7 @@ template <typename T_, int N, int TPT, int TPW, int MODE, class SCH, int... Rs>
 struct Fixed {
     using T = typename FixedElem<T_>::T;
     using ST = Storage<T, typename FixedElem<T_>::S>;
-    static constexpr int PFS = SCH::PFS;
+    static constexpr int PFS = SCH::PFS >= kPersist ? SCH::PFS - kPersist : SCH::PFS;
     static constexpr int MINW = SCH::MINW;
     static constexpr int NST = sizeof...(Rs);
     static constexpr int RAD[NST] = {Rs...};
@@ -162,6 +185,10 @@ struct Fixed {
     }
     static constexpr size_t LDS_BYTES =
         (NST > 1 || MODE != kModeC2C) ? (size_t)STRIDE * EB * TPW : 0;
+    // Persistent and pipelined only where one block fills a CU (see the top of
+    // the file).
+    static constexpr bool PREFETCH =
+        SCH::PFS != kNoPrefetch && (SCH::PFS >= kPersist || LDS_BYTES > kSharedCuLds);
 
     static constexpr int ns_of(int s) {
         int p = 1;
@@ -184,7 +211,7 @@ struct Fixed {
     // 180 -> 145 us at 100000 x 160; with a first radix of 25 that measured
     // the other way round, 211 -> 230 us at 46875 x 400.)
     static constexpr int PF_STAGE =
-        PRE && RAD[0] <= 16 ? 1 : PFS >= 0 ? (PFS < NST ? PFS : NST - 1) : ((NST + PFS) > 0 ? (NST + PFS) : 0);
+        !PREFETCH ? NST : PRE && RAD[0] <= 16 ? 1 : PFS >= 0 ? (PFS < NST ? PFS : NST - 1) : ((NST + PFS) > 0 ? (NST + PFS) : 0);
     static_assert(ns_of(NST) == N, "radices must multiply to N");
     static_assert(!COL || NST >= 2, "column kernels need two stages or more");
 
@@ -373,11 +400,11 @@ struct Fixed {
         if constexpr (!TW_READY) load_tw<S>(a, tb, active, lid);
         if constexpr (PF_HERE) {
             if constexpr (SCH::PF_FIRST) {
-                if (MODE != kModeC2R && g_next >= 0) load0(a, pf, g_next, lid_pf);
+                if (PREFETCH && MODE != kModeC2R && g_next >= 0) load0(a, pf, g_next, lid_pf);
                 load_tw<S + 1>(a, tn, active_n, lid_n);
             } else {
                 load_tw<S + 1>(a, tn, active_n, lid_n);
-                if (MODE != kModeC2R && g_next >= 0) load0(a, pf, g_next, lid_pf);
+                if (PREFETCH && MODE != kModeC2R && g_next >= 0) load0(a, pf, g_next, lid_pf);
             }
         }
         if constexpr (PRE_HERE) {
@@ -736,8 +763,24 @@ struct Fixed {
                 return es != 1 && (((uint32_t)es * DB) & 127u) != 0;
             };
             const bool share = PAIR || NARROW || odd_pitch(a.in_es) || odd_pitch(a.out_es);
-            const int off = share ? (int)xcd_tile(blockIdx.x, (unsigned)G) : (int)blockIdx.x;
+            // (One tile per block: windows of kXcdWindow blocks.  Ranges over
+            // the whole launch would set the XCDs 1/8 of the batch apart, at
+            // equal places of equal rows, which for power-of-two strides are
+            // the same memory channels.)
+            const unsigned win = PREFETCH ? 0u : blockIdx.x / kXcdWindow * kXcdWindow;
+            const unsigned wb = blockIdx.x - win;
+            const unsigned wn =
+                PREFETCH ? (unsigned)G
+                         : ((unsigned)G - win < kXcdWindow ? (unsigned)G - win : kXcdWindow);
+            const int off = (int)(win + (share ? xcd_tile(wb, wn) : wb));
             int grp = off;
+            if constexpr (!PREFETCH) {  // one tile per block
+                load0(a, pf, grp * TPW + slot0, lid0);
+                TwBuf<0> t0;
+                stages_from<0, false>(a, lds_c, grp * TPW, grp * TPW < a.total_slots, slot, lid,
+                                      pf, -1, t0);
+                return;
+            }
             if (grp < ngroups) load0(a, pf, grp * TPW + slot0, lid0);
             for (int w = 0; w < ngroups; w += G, grp += G) {
                 if (grp >= ngroups) break;  // the last window's spare blocks
@@ -747,6 +790,16 @@ struct Fixed {
                 stages_from<0, false>(a, lds_c, grp * TPW, grp * TPW < a.total_slots, slot, lid,
                                       pf, g_next, t0);
             }
+            return;
+        }
+        if constexpr (!PREFETCH) {  // one group of transforms per block
+            const int g = (int)blockIdx.x * TPW + slot;
+            const bool active = g < a.total_slots;
+            if (MODE != kModeC2R) load0(a, pf, g, lid);
+            if constexpr (MODE == kModeC2R) real_pre(a, lds_c, g, active, slot, lid);
+            TwBuf<0> t0;
+            stages_from<0, false>(a, lds_c, g, active, slot, lid, pf, -1, t0);
+            if constexpr (MODE == kModeR2C) real_post(a, lds_c, g, active, slot, lid);
             return;
         }
         int grp = (int)blockIdx.x;
@@ -782,6 +835,7 @@ struct FixedKernel {
                     // 3: the same in wider tiles, for launches that fill the device
     bool paired;    // 2: with the paired modes of real transforms
     int tpt, tpw;
+    int row_tpw, col_tpw;  // 2, 3: columns per block in kModeColRow, kModeColCol
     int nst;
     int radices[kMaxStages];
     size_t lds_bytes;
@@ -805,8 +859,11 @@ hipError_t fixed_launch_one(const void *args, unsigned grid, hipStream_t stream)
     return hipGetLastError();
 }
 
+// Blocks per CU to launch at most: the resident ones of a persistent kernel,
+// any number of the others.
 template <class F>
 int fixed_occupancy() {
+    if (!F::PREFETCH) return 1 << 22;
     int blocks = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, (const void *)k_fixed<F>,
                                                      F::THREADS, F::LDS_BYTES) != hipSuccess) {
@@ -874,14 +931,16 @@ struct FixedReal {
 };
 
 // Registers the column passes of one compile-time plan of column length N
-// (registry kind 2): the first pass of a two-pass plan (kModeColRow), the
-// second (kModeColCol), and with REAL their paired forms for real transforms
-// (kModeColRowPre, kModeColColPost).  KIND 3: a wider tile of the same radices.
-template <typename T, int N, int TPT, int TPW, class SCH, int VARIANT, bool REAL, int KIND,
-          int... Rs>
+// (registry kind 2): the first pass of a two-pass plan (kModeColRow, WR columns
+// per block), the second (kModeColCol, WC), and with REAL their paired forms
+// for real transforms (kModeColRowPre, kModeColColPost, TPW).  KIND 3: a wider
+// tile of the same radices.
+template <typename T, int N, int TPT, int TPW, int WR, int WC, class SCH, int VARIANT, bool REAL,
+          int KIND, int... Rs>
 struct FixedColOf {
     template <int MODE>
-    using F = Fixed<T, N, TPT, TPW, MODE, SCH, Rs...>;
+    using F = Fixed<T, N, TPT, MODE == kModeColRow ? WR : MODE == kModeColCol ? WC : TPW, MODE,
+                    SCH, Rs...>;
     FixedColOf() {
         FixedKernel k{};
         k.n = N;
@@ -891,6 +950,8 @@ struct FixedColOf {
         k.paired = REAL;
         k.tpt = TPT;
         k.tpw = TPW;
+        k.row_tpw = WR;
+        k.col_tpw = WC;
         fixed_fill_radices<Rs...>(k);
         k.lds_bytes = F<kModeColRow>::LDS_BYTES;
         k.launch = [](const void *args, int mode, unsigned grid, hipStream_t s) {
@@ -914,10 +975,10 @@ struct FixedColOf {
         register_fixed(k);
     }
 };
-template <typename T, int N, int TPT, int TPW, class SCH, int VARIANT, int... Rs>
+template <typename T, int N, int TPT, int TPW, int WR, int WC, class SCH, int... Rs>
 using FixedCol =
-    FixedColOf<T, N, TPT, TPW, SCH, VARIANT, std::is_arithmetic<T>::value, 2, Rs...>;
-template <typename T, int N, int TPT, int TPW, class SCH, int VARIANT, int... Rs>
-using FixedColWide = FixedColOf<T, N, TPT, TPW, SCH, VARIANT, false, 3, Rs...>;
+    FixedColOf<T, N, TPT, TPW, WR, WC, SCH, 0, std::is_arithmetic<T>::value, 2, Rs...>;
+template <typename T, int N, int TPT, int TPW, class SCH, int... Rs>
+using FixedColWide = FixedColOf<T, N, TPT, TPW, TPW, TPW, SCH, 0, false, 3, Rs...>;
 
 }  // namespace sfft

@@ -11,10 +11,10 @@ namespace {
 template <class S>
 struct Col16 {
     using E = Stored<S>;
-    const FixedCol<E, 128, 8, 32, Sched<0, 0, 0, 0>, 0, 16, 8> c128;
-    const FixedCol<E, 256, 16, 16, Sched<0, 0, 0, 0>, 0, 16, 16> c256;
-    const FixedCol<E, 512, 32, 16, Sched<0, 0, 0, 0>, 0, 16, 16, 2> c512;
-    const FixedCol<E, 1024, 64, 8, Sched<0, 0, 0, 0>, 0, 16, 16, 4> c1024;
+    const FixedCol<E, 128, 8, 32, 32, 32, Sched<0, 0, 0, 0>, 16, 8> c128;
+    const FixedCol<E, 256, 16, 16, 16, 16, Sched<0, 0, 0, 0>, 16, 16> c256;
+    const FixedCol<E, 512, 32, 16, 16, 16, Sched<0, 0, 0, 0>, 16, 16, 2> c512;
+    const FixedCol<E, 1024, 64, 8, 8, 8, Sched<0, 0, 0, 0>, 16, 16, 4> c1024;
 };
 const Col16<StoreF16> col16_f16;
 const Col16<StoreBF16> col16_bf16;

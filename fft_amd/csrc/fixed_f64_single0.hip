@@ -10,6 +10,9 @@
 // FixedC2C<type, N, threads per transform, transforms per block,
 //          Sched<prefetch stage, min waves per SIMD, pair loads, prefetch first,
 //          LDS pad shift>, variant, radices...>
+// (The rates were measured with persistent kernels; lines with kPersist keep
+// that schedule, 4-20 % faster there than one group per block, and lines with
+// kNoPrefetch the latter above 80 KB of LDS, 7-50 % faster.)
 #include "fixed.h"
 
 namespace sfft {
@@ -20,7 +23,7 @@ const FixedC2C<double, 125, 9, 28, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 5, 5, 5> 
 const FixedC2C<double, 160, 16, 16, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 10> d160;  // 4774 -> 5280
 const FixedC2C<double, 200, 14, 18, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 8, 5, 5> d200;  // 3815 -> 4750
 const FixedC2C<double, 250, 25, 19, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 10, 5, 5> d250;  // 3991 -> 5107
-const FixedC2C<double, 320, 22, 14, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 5, 4> d320;  // 4415 -> 5112
+const FixedC2C<double, 320, 22, 14, Sched<kPersist, 0, 0, 0, kLdsPadShift>, 0, 16, 5, 4> d320;  // 4415 -> 5112
 const FixedC2C<double, 384, 26, 9, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 8, 3> d384;  // 4564 -> 5108
 const FixedC2C<double, 450, 30, 8, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 15, 15, 2> d450;  // 4391 -> 4843
 const FixedC2C<double, 540, 45, 5, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 15, 6, 6> d540;  // 3980 -> 5028
@@ -29,7 +32,7 @@ const FixedC2C<double, 729, 81, 6, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 9, 9, 9> 
 const FixedC2C<double, 810, 90, 2, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 10, 9, 9> d810;  // 3401 -> 4649
 const FixedC2C<double, 972, 108, 2, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 12, 9, 9> d972;  // 3232 -> 4779
 const FixedC2C<double, 1152, 96, 2, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 12, 6> d1152;  // 4161 -> 5215
-const FixedC2C<double, 1280, 86, 3, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 16, 5> d1280;  // 4241 -> 5105
+const FixedC2C<double, 1280, 86, 3, Sched<kPersist, 0, 0, 0, kLdsPadShift>, 0, 16, 16, 5> d1280;  // 4241 -> 5105
 const FixedC2C<double, 1458, 162, 2, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 9, 9, 9, 2> d1458;  // 2525 -> 4070
 const FixedC2C<double, 1620, 180, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 15, 12, 9> d1620;  // 3118 -> 4507
 const FixedC2C<double, 1920, 128, 2, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 15, 8> d1920;  // 4403 -> 5012

@@ -10,6 +10,7 @@
 // FixedC2C<type, N, threads per transform, transforms per block,
 //          Sched<prefetch stage, min waves per SIMD, pair loads, prefetch first,
 //          LDS pad shift>, variant, radices...>
+// (The rates were measured with persistent kernels.)
 #include "fixed.h"
 
 namespace sfft {

@@ -10,6 +10,9 @@
 // FixedC2C<type, N, threads per transform, transforms per block,
 //          Sched<prefetch stage, min waves per SIMD, pair loads, prefetch first,
 //          LDS pad shift>, variant, radices...>
+// (The rates were measured with persistent kernels; lines with kPersist keep
+// that schedule, 4-20 % faster there than one group per block, and lines with
+// kNoPrefetch the latter above 80 KB of LDS, 7-50 % faster.)
 #include "fixed.h"
 
 namespace sfft {
@@ -37,7 +40,7 @@ const FixedC2C<double, 2250, 225, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 15, 15,
 const FixedC2C<double, 2500, 250, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 10, 10, 5, 5> d2500;  // 3343 -> 4860
 const FixedC2C<double, 2880, 240, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 15, 12> d2880;  // 4298 -> 5101
 const FixedC2C<double, 3125, 209, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 5, 5, 5, 5, 5> d3125;  // 3022 -> 3273
-const FixedC2C<double, 3456, 288, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 6, 6, 6> d3456;  // 2546 -> 4870
+const FixedC2C<double, 3456, 288, 1, Sched<kPersist, 0, 0, 0, kLdsPadShift>, 0, 16, 6, 6, 6> d3456;  // 2546 -> 4870
 const FixedC2C<double, 3840, 256, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 16, 15> d3840;  // 4422 -> 4926
 const FixedC2C<double, 4374, 486, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 9, 9, 9, 6> d4374;  // 2296 -> 3696
 const FixedC2C<double, 5000, 500, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 10, 10, 10, 5> d5000;  // 2641 -> 4245

@@ -10,6 +10,9 @@
 // FixedC2C<type, N, threads per transform, transforms per block,
 //          Sched<prefetch stage, min waves per SIMD, pair loads, prefetch first,
 //          LDS pad shift>, variant, radices...>
+// (The rates were measured with persistent kernels; lines with kPersist keep
+// that schedule, 4-20 % faster there than one group per block, and lines with
+// kNoPrefetch the latter above 80 KB of LDS, 7-50 % faster.)
 #include "fixed.h"
 
 namespace sfft {
@@ -36,7 +39,7 @@ const FixedC2C<double, 2025, 135, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 15, 15,
 const FixedC2C<double, 2304, 192, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 12, 12> d2304;  // 3989 -> 5091
 const FixedC2C<double, 2560, 256, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 16, 10> d2560;  // 4146 -> 5165
 const FixedC2C<double, 2916, 324, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 9, 9, 6, 6> d2916;  // 2214 -> 3788
-const FixedC2C<double, 3200, 214, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 8, 5, 5> d3200;  // 3672 -> 4547
+const FixedC2C<double, 3200, 214, 1, Sched<kPersist, 0, 0, 0, kLdsPadShift>, 0, 16, 8, 5, 5> d3200;  // 3672 -> 4547
 const FixedC2C<double, 3600, 240, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 15, 15> d3600;  // 4260 -> 4799
 const FixedC2C<double, 3888, 432, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 12, 9, 6, 6> d3888;  // 2489 -> 4336
 const FixedC2C<double, 4608, 384, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 12, 12, 2> d4608;  // 2459 -> 4268

@@ -13,6 +13,7 @@
 // FixedReal<type, h, threads per transform, transforms per block,
 //           Sched<prefetch stage, min waves per SIMD, pair loads, prefetch first,
 //           LDS pad shift>, variant, radices...>
+// (The rates were measured with persistent kernels.)
 #include "fixed.h"
 
 namespace sfft {

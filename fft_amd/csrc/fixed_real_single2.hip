@@ -13,6 +13,9 @@
 // FixedReal<type, h, threads per transform, transforms per block,
 //           Sched<prefetch stage, min waves per SIMD, pair loads, prefetch first,
 //           LDS pad shift>, variant, radices...>
+// (The rates were measured with persistent kernels; lines with kPersist keep
+// that schedule, 4-20 % faster there than one group per block, and lines with
+// kNoPrefetch the latter above 80 KB of LDS, 7-50 % faster.)
 #include "fixed.h"
 
 namespace sfft {
@@ -39,6 +42,6 @@ const FixedReal<float, 7776, 288, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 32, 9, 
 const FixedReal<float, 9216, 768, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 16, 6, 6> r18432;  // 2053 / 2087 -> 3208 / 2832
 const FixedReal<float, 10368, 864, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 12, 12, 12, 6> r20736;  // 2279 / 2168 -> 2439 / 2811
 const FixedReal<float, 12000, 480, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 32, 25, 15> r24000;  // 2251 / 2111 -> 2724 / 3042
-const FixedReal<float, 14400, 960, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 15, 15, 4> r28800;  // 2364 / 2262 -> 2799 / 2339
+const FixedReal<float, 14400, 960, 1, Sched<kNoPrefetch, 0, 0, 0, kLdsPadShift>, 0, 16, 15, 15, 4> r28800;  // 2364 / 2262 -> 2799 / 2339
 }  // namespace
 }  // namespace sfft

@@ -13,6 +13,9 @@
 // FixedReal<type, h, threads per transform, transforms per block,
 //           Sched<prefetch stage, min waves per SIMD, pair loads, prefetch first,
 //           LDS pad shift>, variant, radices...>
+// (The rates were measured with persistent kernels; lines with kPersist keep
+// that schedule, 4-20 % faster there than one group per block, and lines with
+// kNoPrefetch the latter above 80 KB of LDS, 7-50 % faster.)
 #include "fixed.h"
 
 namespace sfft {
@@ -39,6 +42,6 @@ const FixedReal<float, 8000, 320, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 32, 25,
 const FixedReal<float, 9600, 640, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 15, 8, 5> r19200;  // 2129 / 2147 -> 3079 / 2953
 const FixedReal<float, 10800, 720, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 15, 15, 3> r21600;  // 2206 / 2127 -> 3068 / 2891
 const FixedReal<float, 12288, 512, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 32, 32, 12> r24576;  // 2338 / 2215 -> 2885 / 2911
-const FixedReal<float, 15360, 1024, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 16, 15, 4> r30720;  // 2532 / 2395 -> 2889 / 3106
+const FixedReal<float, 15360, 1024, 1, Sched<kNoPrefetch, 0, 0, 0, kLdsPadShift>, 0, 16, 16, 15, 4> r30720;  // 2532 / 2395 -> 2889 / 3106
 }  // namespace
 }  // namespace sfft

@@ -15,6 +15,9 @@
 // FixedC2C<type, N, threads per transform, transforms per block,
 //          Sched<prefetch stage, min waves per SIMD, pair loads, prefetch first,
 //          LDS pad shift>, variant, radices...>
+// (The rates were measured with persistent kernels; lines with kPersist keep
+// that schedule, 4-20 % faster there than one group per block, and lines with
+// kNoPrefetch the latter above 80 KB of LDS, 7-50 % faster.)
 #include "fixed.h"
 
 namespace sfft {
@@ -36,13 +39,13 @@ const FixedC2C<float, 4320, 160, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 32, 15, 
 const FixedC2C<float, 4800, 160, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 32, 15, 10> c4800;  // 2699 -> 4347
 const FixedC2C<float, 5400, 360, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 15, 15, 8, 3> c5400;  // 2795 -> 3300
 const FixedC2C<float, 6000, 400, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 25, 16, 15> c6000;  // 3631 -> 4166
-const FixedC2C<float, 6400, 256, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 32, 25, 8> c6400;  // 3649 -> 4520
-const FixedC2C<float, 7200, 240, 1, Sched<0, 0, 0, 0, kLdsPadShift, 3>, 0, 32, 15, 15> c7200;  // 3394 -> 4331
+const FixedC2C<float, 6400, 256, 1, Sched<kPersist, 0, 0, 0, kLdsPadShift>, 0, 32, 25, 8> c6400;  // 3649 -> 4520
+const FixedC2C<float, 7200, 240, 1, Sched<kPersist, 0, 0, 0, kLdsPadShift, 3>, 0, 32, 15, 15> c7200;  // 3394 -> 4331
 const FixedC2C<float, 8000, 320, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 32, 25, 10> c8000;  // 2433 -> 3788
 const FixedC2C<float, 9216, 768, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 16, 6, 6> c9216;  // 2393 -> 3904
 const FixedC2C<float, 10240, 683, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 16, 8, 5> c10240;  // 2426 -> 3817
 const FixedC2C<float, 11664, 432, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 9, 9, 9> c11664;  // 1962 -> 3545
 const FixedC2C<float, 12960, 480, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 32, 9, 9, 5> c12960;  // 1917 -> 3446
-const FixedC2C<float, 19200, 640, 1, Sched<0, 0, 0, 0, kLdsPadShift, 3>, 0, 32, 10, 10, 6> c19200;  // 1818 -> 2153
+const FixedC2C<float, 19200, 640, 1, Sched<kNoPrefetch, 0, 0, 0, kLdsPadShift, 3>, 0, 32, 10, 10, 6> c19200;  // 1818 -> 2153
 }  // namespace
 }  // namespace sfft

@@ -15,6 +15,9 @@
 // FixedC2C<type, N, threads per transform, transforms per block,
 //          Sched<prefetch stage, min waves per SIMD, pair loads, prefetch first,
 //          LDS pad shift>, variant, radices...>
+// (The rates were measured with persistent kernels; lines with kPersist keep
+// that schedule, 4-20 % faster there than one group per block, and lines with
+// kNoPrefetch the latter above 80 KB of LDS, 7-50 % faster.)
 #include "fixed.h"
 
 namespace sfft {
@@ -42,6 +45,6 @@ const FixedC2C<float, 8748, 972, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 12, 9, 9
 const FixedC2C<float, 10125, 675, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 15, 15, 15, 3> c10125;  // 2434 -> 2876
 const FixedC2C<float, 11520, 768, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 16, 15, 3> c11520;  // 2508 -> 3740
 const FixedC2C<float, 12800, 512, 1, Sched<0, 0, 0, 0, kLdsPadShift, 3>, 0, 32, 25, 16> c12800;  // 2398 -> 3399
-const FixedC2C<float, 17280, 576, 1, Sched<0, 0, 0, 0, kLdsPadShift, 3>, 0, 32, 15, 6, 6> c17280;  // 1886 -> 2038
+const FixedC2C<float, 17280, 576, 1, Sched<kNoPrefetch, 0, 0, 0, kLdsPadShift, 3>, 0, 32, 15, 6, 6> c17280;  // 1886 -> 2038
 }  // namespace
 }  // namespace sfft
