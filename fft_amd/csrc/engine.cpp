@@ -180,6 +180,7 @@ constexpr size_t kTwoPassFrom = 16000;
 // 1.06-1.20x over the previous choice); a final re-sweep of all of them with
 // the final kernels set ten more (31104, 32400, 36864, 46080, 48600, 54000,
 // 55296, 147456, 184320, 196608: 1.07-1.17x).
+// 2^18 takes 256 x 1024 (both directions of 2^18 x 64: 236 -> 221 us).
 // The last two, 2^21 and 2^22, measured 3-5 % faster with first-pass
 // columns of 4096 in two runs each (2^21 x 8: 1.69-1.74 -> 1.79-1.81;
 // 2^22 x 4: 1.64-1.70 -> 1.74).  Sorted by length.
@@ -203,8 +204,8 @@ static const MeasuredSplit kMeasuredSplits[] = {
     {140625, 625}, {144000, 288}, {145800, 729}, {147456, 144}, {155520, 360}, {156250, 625},
     {157464, 729}, {163840, 160}, {164025, 729}, {174960, 432}, {180000, 288}, {182250, 375},
     {184320, 360}, {196608, 192}, {202500, 500}, {204800, 1024}, {216000, 432}, {218700, 729},
-    {225000, 360}, {243000, 500}, {245760, 1024}, {248832, 512}, {253125, 625}, {2097152, 4096},
-    {4194304, 4096},
+    {225000, 360}, {243000, 500}, {245760, 1024}, {248832, 512}, {253125, 625}, {262144, 256},
+    {2097152, 4096}, {4194304, 4096},
 };
 
 // The same for real FP32 two-pass plans (RealFFT, not the half-bin shifted
@@ -238,21 +239,20 @@ static const MeasuredSplit kMeasuredRealSplits[] = {
 };
 
 // The same for the power-of-two two-pass lengths of the other precisions
-// (complex, about 128 MB per launch, every split timed twice; listed where
-// both timings beat both of the scored split's by more than 5 %, and at 2^20
-// for 16-bit storage and F32X, where 2^20 x 16 measured f16 110-113 -> 105-106
-// us and F32X 222-225 -> 196 us).  16-bit storage (IEEE half and bfloat16:
-// 2^18 1.16-1.22x, 2^19 1.11-1.18x, 2^21 1.07-1.08x):
+// (complex, every split timed forward and inverse over 134 MB (16-bit: 67 MB)
+// of input; listed where it beats the scored split).  16-bit storage (IEEE half
+// and bfloat16; 2^18 180 -> 155 us, 2^19 192 -> 177, 2^20 x 16 196 -> 194 and
+// without a wide tile at one transform, 2^21 as before):
 static const MeasuredSplit kMeasuredSplits16[] = {
     {262144, 2048}, {524288, 2048}, {1048576, 4096}, {2097152, 2048},
 };
-// FP32 storage under FP64 arithmetic (F32X; 2^19 1.13x):
+// FP32 storage under FP64 arithmetic (F32X; 2^17 311 -> 279 us, 2^19 370 -> 355):
 static const MeasuredSplit kMeasuredSplitsF32X[] = {
-    {524288, 2048}, {1048576, 4096},
+    {131072, 512}, {524288, 512}, {1048576, 4096},
 };
-// FP64 (2^21 1.17x, 2^22 1.10x):
+// FP64 (2^21 626 -> 522 us, 2^22 716 -> 585, against first passes of 4096):
 static const MeasuredSplit kMeasuredSplitsF64[] = {
-    {2097152, 4096}, {4194304, 4096},
+    {2097152, 1024}, {4194304, 2048},
 };
 
 template <size_t K>
@@ -377,10 +377,6 @@ static bool layout_columns(int n, int prec, int max_cols, const PlanHints *h, Pa
 static void use_fixed_columns(PassPlan &pp, size_t n, int prec, int mode, bool real) {
     const FixedKernel *fk = find_fixed((int)n, prec, 2, -1);
     if (!fk) return;
-    // FP64 compiled columns measured faster than the runtime-planned pass
-    // only with 512 or more columns per transform (2^18 = 512 x 512: 1.81
-    // -> 2.26 TB/s; 2^16 = 128 x 512: 2.47 runtime-planned, 2.13 compiled)
-    if (arith_f64(prec) && pp.slots_per_transform < 512) return;
     std::vector<int> rs(fk->radices, fk->radices + fk->nst);
     int ept = 0;
     for (int e : {kEptSmall, kEptLarge})

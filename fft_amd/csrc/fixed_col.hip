@@ -1,5 +1,5 @@
 // fixed_col.hip -- compile-time column passes of two-pass plans, complex
-// FP32 and FP64.  FixedCol<type, column length N, threads per column,
+// FP32, FP64 and F32X.  FixedCol<type, column length N, threads per column,
 // columns per block in the paired modes, in the first pass, in the second,
 // Sched<...>, radices...>; a two-pass plan whose column length has one uses it
 // for that pass (same radices as the runtime-planned pass, so the same bits).
@@ -21,8 +21,23 @@ const FixedCol<float, 512, 32, 16, 16, 8, Sched<0, 0, 0, 0, kLdsPadShift, 1>, 16
 const FixedCol<float, 1024, 64, 8, 8, 8, Sched<0, 0, 0, 0, kLdsPadShift, 1>, 16, 16, 4> col1024;
 const FixedCol<float, 2048, 128, 8, 8, 4, Sched<kNoPrefetch, 0, 0, 0, kLdsPadShift, 1>, 16, 16, 8>
     col2048;
-// FP64 (16-byte values: half the columns per LDS budget)
+// FP64 (16-byte values; 256 MB per launch with 256 columns, first / second
+// pass, runtime-planned pass -> here): 128 103/87 -> 93/80 us, 256 107/87 ->
+// 97/82, 512 121/95 -> 113/89, 1024 158/133 -> 135/111, 2048 198/155 -> 163/138.
+// 172 registers, two waves per SIMD: a third (168 registers) spilled, 111 -> 128
+// us in the second pass of 1024.
+const FixedCol<double, 128, 8, 16, 16, 16, Sched<0, 0, 0, 0, kLdsPadShift, 1>, 16, 8> col128d;
+const FixedCol<double, 256, 16, 16, 16, 16, Sched<0, 0, 0, 0, kLdsPadShift, 1>, 16, 16> col256d;
 const FixedCol<double, 512, 32, 8, 8, 8, Sched<0, 0, 0, 0, kLdsPadShift, 1>, 16, 16, 2> col512d;
 const FixedCol<double, 1024, 64, 4, 4, 4, Sched<0, 0, 0, 0, kLdsPadShift, 1>, 16, 16, 4> col1024d;
+const FixedCol<double, 2048, 128, 4, 4, 4, Sched<kNoPrefetch, 0, 0, 0, kLdsPadShift, 1>, 16, 16, 8>
+    col2048d;
+// FP32 storage under FP64 arithmetic: the same shapes
+using X = Stored<StoreF32>;
+const FixedCol<X, 128, 8, 16, 16, 16, Sched<0, 0, 0, 0>, 16, 8> col128x;
+const FixedCol<X, 256, 16, 16, 16, 16, Sched<0, 0, 0, 0>, 16, 16> col256x;
+const FixedCol<X, 512, 32, 8, 8, 8, Sched<0, 0, 0, 0>, 16, 16, 2> col512x;
+const FixedCol<X, 1024, 64, 4, 4, 4, Sched<0, 0, 0, 0>, 16, 16, 4> col1024x;
+const FixedCol<X, 2048, 128, 4, 4, 4, Sched<kNoPrefetch, 0, 0, 0>, 16, 16, 8> col2048x;
 }  // namespace
 }  // namespace sfft
