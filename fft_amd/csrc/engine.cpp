@@ -244,7 +244,7 @@ static const MeasuredSplit kMeasuredRealSplits[] = {
 // and bfloat16; 2^18 180 -> 155 us, 2^19 192 -> 177, 2^20 x 16 196 -> 194 and
 // without a wide tile at one transform, 2^21 as before):
 static const MeasuredSplit kMeasuredSplits16[] = {
-    {262144, 2048}, {524288, 2048}, {1048576, 4096}, {2097152, 2048},
+    {262144, 256}, {524288, 512}, {1048576, 1024}, {2097152, 2048},
 };
 // FP32 storage under FP64 arithmetic (F32X; 2^17 311 -> 279 us, 2^19 370 -> 355):
 static const MeasuredSplit kMeasuredSplitsF32X[] = {
@@ -832,6 +832,7 @@ void Plan::build_tables() {
     } else if (passes_.size() > 1) {
         int shift = 0;
         while ((1ull << (2 * shift)) < cn_) ++shift;
+        if (sizeof(T) == 4 && cn_ <= (1u << 24)) shift = std::min(shift, kFineShift);
         ptw_shift_ = shift;
         const size_t nf = 1ull << shift, nc = (cn_ + nf - 1) >> shift;
         alloc(&d_ptw_fine_, nf * sizeof(C2<T>));

@@ -57,6 +57,10 @@ template <typename T>
 hipError_t gen_real_twiddles(C2<T> *tmi, C2<T> *rot, size_t n, int half_shift,
                              hipStream_t stream);
 
+// Largest fine table (2^kFineShift entries) that the wide column kernels keep
+// in LDS; FP32 plans up to 2^24 values stay within it.
+constexpr int kFineShift = 11;
+
 // Two-level table for W_N^m: fine[m] for m < 2^shift,
 // coarse[q] = W_N^{q 2^shift} for q < ceil(N / 2^shift); computed in FP64,
 // rounded once to T.
