@@ -30,8 +30,12 @@ _REAL = {torch.float32: L.F32, torch.float64: L.F64}
 
 
 def _stream_handle(stream=None) -> int:
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return s.cuda_stream
+    """hipStream_t of `stream`, or of the current stream of the current device
+    (read without building a Stream object: 0.1 us instead of 2.8, of 7.9 us
+    for a whole fft() call)."""
+    if stream is not None:
+        return stream.cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 class Plan:
@@ -88,8 +92,10 @@ class Plan:
 
     def execute_ptr(self, in_ptr: int, out_ptr: int, batch: int, direction: int,
                     stream_handle: int) -> None:
-        L.check(L.lib().sfft_execute(self._h, ctypes.c_void_p(in_ptr), ctypes.c_void_p(out_ptr),
-                                     batch, direction, ctypes.c_void_p(stream_handle)))
+        # (the entry point's argument types turn the addresses into pointers)
+        rc = L.lib().sfft_execute(self._h, in_ptr, out_ptr, batch, direction, stream_handle)
+        if rc:
+            L.check(rc)
 
     def workspace_size(self, batch: int, in_place: bool) -> int:
         """Device workspace bytes an execute call needs (sfft_plan_workspace_size)."""
