@@ -518,13 +518,13 @@ Plan::Plan(size_t n, int kind, int prec, const PlanHints *h) : n_(n), kind_(kind
         const size_t max_cols = (h && h->tpw) ? (size_t)h->tpw : 8;
         // the measured split where the table has one (if its layout fails,
         // the scored search runs over every split)
-        auto search = [&](size_t only_n1) {
+        auto search = [&](size_t only_n1, bool compiled) {
             for (size_t n1 = 32; n1 * 16 <= cn_; ++n1) {
                 if (cn_ % n1) continue;
                 if (h && h->split > 1 && n1 != h->split) continue;
                 if (only_n1 && n1 != only_n1) continue;
                 const size_t n2 = cn_ / n1;
-                if (compiled_split &&
+                if (compiled &&
                     (!find_fixed((int)n1, prec, 2, -1) || !find_fixed((int)n2, prec, 2, -1)))
                     continue;
                 PassPlan p1, p2;
@@ -554,8 +554,14 @@ Plan::Plan(size_t n, int kind, int prec, const PlanHints *h) : n_(n), kind_(kind
                        : prec == kF32X ? lookup_split(kMeasuredSplitsF32X, cn_)
                        : prec == kF64  ? lookup_split(kMeasuredSplitsF64, cn_)
                                        : 0;
-        search(table_n1);
-        if (!best_n1 && table_n1) search(0);
+        // a split of two compiled column lengths where there is one (FP32 and
+        // FP64, 128 MB batches, against the scored split with its runtime-planned
+        // passes: 331776 172 -> 110 us, 1000000 188 -> 144, FP64 708588
+        // 180 -> 140, R2C 839808 270 -> 180), else any
+        const bool prefer = free_split && (prec == kF32 || prec == kF64);
+        if (table_n1) search(table_n1, compiled_split);
+        if (!best_n1 && (compiled_split || prefer)) search(0, true);
+        if (!best_n1 && !compiled_split) search(0, false);
         if (!best_n1 && !ok)
             throw Error(SFFT_ERR_UNSUPPORTED_SIZE,
                         "size " + std::to_string(n) + ": no two-pass split fits LDS (F64 plans "
