@@ -8,8 +8,8 @@
 // about 256 threads per block.  A length is listed only where its faster
 // candidate beat the runtime pass by 5 % or more over both directions, with
 // neither direction 3 % slower (forward / inverse GB/s, runtime -> compiled,
-// follow each line).  The other lengths keep the runtime pass (their
-// candidates lost, up to 2.5x slower above h = 10000).
+// follow each line).  The lengths whose candidates lost then run one group per
+// block, in fixed_real_single4.hip to fixed_real_single11.hip.
 // FixedReal<type, h, threads per transform, transforms per block,
 //           Sched<prefetch stage, min waves per SIMD, pair loads, prefetch first,
 //           LDS pad shift>, variant, radices...>

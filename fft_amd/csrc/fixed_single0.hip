@@ -6,10 +6,9 @@
 // (radix 32 allowed), threads per transform as that model computes them, and
 // about 256 threads per block.  A length is listed only where its faster
 // candidate beat the runtime pass by 5 % or more (the rate pair in GB/s, runtime
-// -> compiled, follows each line).  Lengths where the candidates lost (up to
-// 2.4x slower, mostly lengths above 10000 at 600 to 1000 threads per
-// transform) keep the runtime pass.  Lines whose schedule ends in 3 use
-// non-temporal input loads and output stores (Sched NT): 800, 1536, 1728,
+// -> compiled, follows each line).  The lengths whose candidates lost then run
+// one group per block, in fixed_single4.hip to fixed_single7.hip.  Lines whose
+// schedule ends in 3 use non-temporal input loads and output stores (Sched NT): 800, 1536, 1728,
 // 2160, 2430, 2560, 3072, 7200, 7680, 12288, 12800, 17280 and 19200 measured
 // 7-18 % faster with them, others up to 2.5x slower.
 // FixedC2C<type, N, threads per transform, transforms per block,
