@@ -6,7 +6,8 @@
 // to it), at its threads per block and at twice as many transforms per
 // block.  A length is listed only where the faster candidate beat the runtime
 // pass by 5 % or more (the rate pair in GB/s, runtime -> compiled, follows
-// each line); the others keep the runtime pass.
+// each line); the others run one group per block, in fixed_f64_single4.hip and
+// fixed_f64_single5.hip.
 // FixedC2C<type, N, threads per transform, transforms per block,
 //          Sched<prefetch stage, min waves per SIMD, pair loads, prefetch first,
 //          LDS pad shift>, variant, radices...>
