@@ -558,7 +558,7 @@ Plan::Plan(size_t n, int kind, int prec, const PlanHints *h) : n_(n), kind_(kind
         // FP64, 128 MB batches, against the scored split with its runtime-planned
         // passes: 331776 172 -> 110 us, 1000000 188 -> 144, FP64 708588
         // 180 -> 140, R2C 839808 270 -> 180), else any
-        const bool prefer = free_split && (prec == kF32 || prec == kF64);
+        const bool prefer = free_split;
         if (table_n1) search(table_n1, compiled_split);
         if (!best_n1 && (compiled_split || prefer)) search(0, true);
         if (!best_n1 && !compiled_split) search(0, false);
