@@ -394,8 +394,10 @@ static void use_fixed_columns(PassPlan &pp, size_t n, int prec, int mode, bool r
     pp.fixed = fk;
     pp.fixed_grid[mode] = (unsigned)(fk->blocks_per_cu(mode) * device_info().cu_count);
     if (real && fk->paired) {
-        const int pm = mode == kModeColRow ? kModeColRowPre : kModeColColPost;
-        pp.fixed_grid[pm] = (unsigned)(fk->blocks_per_cu(pm) * device_info().cu_count);
+        const bool first = mode == kModeColRow;
+        for (int m : {first ? kModeColRowPre : kModeColColPost,
+                      first ? kModeColRowRot : kModeColColRot})
+            pp.fixed_grid[m] = (unsigned)(fk->blocks_per_cu(m) * device_info().cu_count);
     }
 }
 
@@ -945,7 +947,9 @@ void Plan::run(const void *in, size_t in_dist, void *out, size_t out_dist, size_
 
 // Columns per block of a column kernel in a mode.
 static int column_tile(const FixedKernel &fk, int mode) {
-    return mode == kModeColRow ? fk.row_tpw : mode == kModeColCol ? fk.col_tpw : fk.tpw;
+    return mode == kModeColRow || mode == kModeColRowRot   ? fk.row_tpw
+           : mode == kModeColCol || mode == kModeColColRot ? fk.col_tpw
+                                                           : fk.tpw;
 }
 
 static int plain_column_mode(size_t p) { return p == 0 ? kModeColRow : kModeColCol; }
@@ -1046,9 +1050,8 @@ void Plan::run_fixed(const void *in, void *out, size_t batch, int inverse,
 }
 template void Plan::run_fixed<float>(const void *, void *, size_t, int, hipStream_t) const;
 
-// Compiled column kernels run plain column passes (complex ones, and real ones
-// with no rotation at their loads or stores) and the paired passes of real
-// transforms; -1 otherwise.
+// Compiled column kernels run plain column passes, and the paired and rotating
+// passes of real transforms; -1 otherwise.
 int Plan::column_mode(size_t p, int inverse) const {
     const PassPlan &pp = passes_[p];
     if (passes_.size() != 2) return -1;
@@ -1059,7 +1062,9 @@ int Plan::column_mode(size_t p, int inverse) const {
         if (pp.fixed && pp.fixed_grid[pm]) return pm;
         return p == 0 ? -1 : plain;
     }
-    return kind_ == kR2CHalf ? -1 : plain;
+    if (kind_ != kR2CHalf) return plain;
+    const int rm = p == 0 ? kModeColRowRot : kModeColColRot;
+    return pp.fixed && pp.fixed_grid[rm] ? rm : -1;
 }
 
 // Pass p of a two-pass plan through its compiled column kernel.  The
@@ -1100,6 +1105,7 @@ void Plan::run_fixed_columns(size_t p, const FixedKernel &fk, int mode, unsigned
         if (paired) a.tiles = make_fastdiv(tiles);
         a.real_tw = (const C2<T> *)d_real_tw_;
         a.half_shift = kind_ == kR2CHalf;
+        a.rot = (const C2<T> *)d_rot_;
         a.in_bs = (int32_t)dsrc;
         a.in_ss = (int32_t)pp.in_slot_stride;
         a.in_es = (int32_t)pp.in_elem_stride;

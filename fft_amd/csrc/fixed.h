@@ -112,6 +112,16 @@ struct Sched {
     static constexpr int PF_FIRST = PF_FIRST_;
     static constexpr int PADSH = PADSH_;
     static constexpr int NT = NT_;
+    static constexpr bool ROT = false;
+};
+// Column passes that also rotate (half-bin shifted real transforms): the
+// rotations are read as the data is, from a table of one transform.  Kernels of
+// their own, because the branch alone cost the plain 1024 pass 20 % (2^20 x 16
+// 125 -> 160 us).  Against the runtime-planned pass, both directions of 128 MB
+// batches: 1.1-1.4x (218700 397 -> 286 us, FP64 100000 355 -> 255).
+template <class S>
+struct Rotated : S {
+    static constexpr bool ROT = true;
 };
 
 // Element type of a compiled kernel: float / double (stored as is), or
@@ -428,6 +438,20 @@ struct Fixed {
                     }
                 }
             }
+            if constexpr (SCH::ROT && MODE == kModeColRow) {
+                uint32_t t, c;
+                column_of(a, g, t, c);
+#pragma unroll
+                for (int b = 0; b < B; ++b) {
+                    const uint32_t j = (uint32_t)(lid + b * TPT);
+                    if (active && jvalid(b)) {
+#pragma unroll
+                        for (int r = 0; r < R; ++r)
+                            v[b][r] = cmul(v[b][r], a.rot[c + (j + (uint32_t)(r * NB)) *
+                                                                  (uint32_t)a.in_es]);
+                    }
+                }
+            }
         } else {
 #pragma unroll
             for (int b = 0; b < B; ++b) {
@@ -490,6 +514,19 @@ struct Fixed {
             for (int b = 0; b < B; ++b)
 #pragma unroll
                 for (int t2 = 0; t2 < R; ++t2) flip_im(v[b][t2], a.flip_out);
+            if constexpr (SCH::ROT && COL_OUT) {
+#pragma unroll
+                for (int b = 0; b < B; ++b) {
+                    const int j = lid + b * TPT;
+                    if (active && jvalid(b)) {
+                        const int o = (j / NS) * NS * R + j % NS;
+#pragma unroll
+                        for (int t2 = 0; t2 < R; ++t2)
+                            v[b][t2] = cmulc(v[b][t2], a.rot[c + (uint32_t)(o + t2 * NS) *
+                                                                     (uint32_t)a.out_es]);
+                    }
+                }
+            }
             if (a.post_tw && a.ptw_full) {
                 // the four-step factors from the full table: the lanes of a
                 // slot read consecutive entries (lanes without a butterfly
@@ -940,14 +977,17 @@ struct FixedReal {
 // Registers the column passes of one compile-time plan of column length N
 // (registry kind 2): the first pass of a two-pass plan (kModeColRow, WR columns
 // per block), the second (kModeColCol, WC), and with REAL their paired forms
-// for real transforms (kModeColRowPre, kModeColColPost, TPW).  KIND 3: a wider
-// tile of the same radices.
+// for real transforms (kModeColRowPre, kModeColColPost, TPW) and the rotating
+// ones (kModeColRowRot, kModeColColRot: the plain passes' tiles).  KIND 3: a
+// wider tile of the same radices.
 template <typename T, int N, int TPT, int TPW, int WR, int WC, class SCH, int VARIANT, bool REAL,
           int KIND, int... Rs>
 struct FixedColOf {
     template <int MODE>
     using F = Fixed<T, N, TPT, MODE == kModeColRow ? WR : MODE == kModeColCol ? WC : TPW, MODE,
                     SCH, Rs...>;
+    template <int MODE>
+    using FRot = Fixed<T, N, TPT, MODE == kModeColRow ? WR : WC, MODE, Rotated<SCH>, Rs...>;
     FixedColOf() {
         FixedKernel k{};
         k.n = N;
@@ -967,6 +1007,10 @@ struct FixedColOf {
                     return fixed_launch_one<F<kModeColRowPre>>(args, grid, s);
                 if (mode == kModeColColPost)
                     return fixed_launch_one<F<kModeColColPost>>(args, grid, s);
+                if (mode == kModeColRowRot)
+                    return fixed_launch_one<FRot<kModeColRow>>(args, grid, s);
+                if (mode == kModeColColRot)
+                    return fixed_launch_one<FRot<kModeColCol>>(args, grid, s);
             }
             return mode == kModeColCol ? fixed_launch_one<F<kModeColCol>>(args, grid, s)
                                        : fixed_launch_one<F<kModeColRow>>(args, grid, s);
@@ -975,6 +1019,8 @@ struct FixedColOf {
             if constexpr (REAL) {
                 if (mode == kModeColRowPre) return fixed_occupancy<F<kModeColRowPre>>();
                 if (mode == kModeColColPost) return fixed_occupancy<F<kModeColColPost>>();
+                if (mode == kModeColRowRot) return fixed_occupancy<FRot<kModeColRow>>();
+                if (mode == kModeColColRot) return fixed_occupancy<FRot<kModeColCol>>();
             }
             return mode == kModeColCol ? fixed_occupancy<F<kModeColCol>>()
                                        : fixed_occupancy<F<kModeColRow>>();

@@ -66,8 +66,11 @@ enum : int32_t {
     // a tile holds columns and their mirror images
     kModeColRowPre = 8,   // first pass, inverse: pre-process at the column loads
     kModeColColPost = 9,  // second pass, forward: post-process at the column stores
+    // the plain passes with the half-bin shift's rotation
+    kModeColRowRot = 10,  // first pass, forward: at the column loads
+    kModeColColRot = 11,  // second pass, inverse: at the column stores
 };
-constexpr int kModes = 10;
+constexpr int kModes = 12;
 
 // The pair loops of the real pre-/post-process (signalsmith-fft.h:463-472,
 // :482-492) visit i = 0..h/2 (1..h/2 without the half shift) with partner
