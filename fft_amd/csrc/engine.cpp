@@ -444,7 +444,7 @@ Plan::Plan(size_t n, int kind, int prec, const PlanHints *h) : n_(n), kind_(kind
             throw Error(SFFT_ERR_UNSUPPORTED_SIZE, "size " + std::to_string(n) + " too large");
         // one launch where a compiled convolution length fits LDS, three
         // where it is a compiled column length times a compiled row length
-        // (100003 x 64, both directions: 639 us as the launch sequence, 292 us), the launch
+        // (100003 x 64, both directions: 639 us as the launch sequence, 270 us), the launch
         // sequence beyond (M above 240 x 16384 in F32, 240 x 8192 in F64)
         bs_row_ = bluestein_length(cn_);
         chirp_ = find_chirp(cn_, prec == kF64 ? 1 : 0);
