@@ -23,7 +23,7 @@
 //    half of its elements.
 //  - Twiddles of a stage are loaded before the exchange that feeds it.
 // Measured (N = 1009, 4096 transforms, M = 2048, F32; forward and inverse
-// together, 132 MB): 270 us as separate launches, 74 us here; 521 -> 83 us for
+// together, 132 MB): 270 us as separate launches, 66 us here; 521 -> 72 us for
 // a first call, which no longer allocates its workspace.
 //
 // Longer lengths take M = N1 N2 and three launches over a workspace of M

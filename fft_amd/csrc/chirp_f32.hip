@@ -1,12 +1,16 @@
 // chirp_f32.hip -- one-launch chirp-z kernels, FP32: convolution lengths up
 // to 4096.  ChirpReg<type, rows of a longer one, M, threads per transform,
-// transforms per block, minimum waves per SIMD, radices...>: R b R with M / R
-// threads, one radix-R butterfly each.  These kernels are bound by vector
+// transforms per block, minimum waves per SIMD, radices...>: mostly R b R
+// with M / R threads, one radix-R butterfly each.  These kernels are bound by vector
 // instructions (about 100 per element of M), so a length is listed only where
 // it beat the next power of two: 1280, 1792, 2560 and 3840 did not (6.2 to 9.7
 // ps per element of M against 4.9 at 1024 and 2048, at 8 to 16 transforms
 // resident per CU).  Two transforms per thread, which halves the table loads,
 // measured 0.62-0.98x: half the resident waves.
+// 1024, 2048 and 4096 take eight elements a thread and one more stage, which
+// halves a wave's registers and LDS (twice the waves).  Both directions, sixteen
+// / eight: 509 x 8192 68.2 / 64.8 us, 1009 x 4096 73.4 / 68.2, x 20000 376 / 321,
+// 1999 x 2048 75.6 / 73.5, and one transform of 1009 17.1 / 11.3.
 #include "chirp.h"
 
 namespace sfft {
@@ -21,10 +25,10 @@ const ChirpReg<float, false, 448, 56, 4, 4, 8, 7, 8> c448;
 const ChirpReg<float, false, 512, 64, 4, 4, 8, 8, 8> c512;
 const ChirpReg<float, false, 640, 80, 4, 4, 8, 10, 8> c640;
 const ChirpReg<float, false, 768, 48, 4, 4, 16, 3, 16> c768;
-const ChirpReg<float, false, 1024, 64, 4, 4, 16, 4, 16> c1024;
+const ChirpReg<float, false, 1024, 128, 2, 4, 8, 4, 4, 8> c1024;
 const ChirpReg<float, false, 1536, 96, 2, 3, 16, 6, 16> c1536;
-const ChirpReg<float, false, 2048, 128, 2, 4, 16, 8, 16> c2048;
+const ChirpReg<float, false, 2048, 256, 1, 4, 8, 8, 4, 8> c2048;
 const ChirpReg<float, false, 3072, 256, 1, 4, 16, 16, 12> c3072;
-const ChirpReg<float, false, 4096, 256, 1, 4, 16, 16, 16> c4096;
+const ChirpReg<float, false, 4096, 512, 1, 4, 8, 8, 8, 8> c4096;
 }  // namespace
 }  // namespace sfft

@@ -45,12 +45,15 @@ def _edges(ms):
 
 N1 = [128, 144, 160, 176, 192, 208, 240]
 # (M, n) of plans of three launches: the largest chirp-z n of N1 x 128 and of
-# N1 x 1024 (F64: 64 and 512), the first one past one launch, and the ends
+# N1 x 1024 (F64: 64 and 512), the first one past one launch, one of each row
+# length of eight elements a thread, and the ends
 S32 = _edges([16384] + [c * 128 for c in N1[1:]])[2:] + \
     [(c * 1024, _edges([c * 1024])[-1][1]) for c in N1[::2]] + \
+    [(m, _edges([m])[-1][1]) for m in (208 * 2048, 208 * 4096)] + \
     [(240 << 14, 1966080 - 1)]
 S64 = _edges([8192] + [c * 64 for c in N1[1:]])[2:] + \
-    [(c * 512, _edges([c * 512])[-1][1]) for c in N1[1::2]] + [(240 << 13, 983040 - 1)]
+    [(c * 512, _edges([c * 512])[-1][1]) for c in N1[1::2]] + \
+    [(m, _edges([m])[-1][1]) for m in (208 * 1024, 208 * 2048)] + [(240 << 13, 983040 - 1)]
 
 
 def _stream():
