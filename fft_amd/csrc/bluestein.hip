@@ -45,14 +45,6 @@ __global__ void k_bs_scale(C2<T> *z, uint64_t m_len, T s) {
         z[m] = {z[m].x * s, z[m].y * s};
 }
 
-template <typename T>
-__global__ void k_bs_digit_swap(const C2<T> *src, C2<T> *dst, uint64_t n1, uint64_t m_len) {
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    const uint64_t n2 = m_len / n1;
-    for (uint64_t m = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; m < m_len; m += stride)
-        dst[m] = src[m / n2 + n1 * (m % n2)];
-}
-
 // a[b][m] = load(x[b], m) * w[m] for m < N, 0 up to M.  The load applies the
 // conjugation of the inverse, the half-bin rotation of a forward
 // ModifiedRealFFT, or the real inverse pre-process of bin m.
@@ -125,8 +117,9 @@ static dim3 grid_rows(uint64_t len, uint64_t batch) {
 template <typename T>
 hipError_t bs_gen_chirp(C2<T> *w, C2<T> *b, size_t n_len, size_t m_len, hipStream_t stream) {
     hipLaunchKernelGGL((k_bs_chirp<T>), grid_1d(n_len), dim3(256), 0, stream, w, (uint64_t)n_len);
-    hipLaunchKernelGGL((k_bs_kernel<T>), grid_1d(m_len), dim3(256), 0, stream, b, (const C2<T> *)w,
-                       (uint64_t)n_len, (uint64_t)m_len);
+    if (b)
+        hipLaunchKernelGGL((k_bs_kernel<T>), grid_1d(m_len), dim3(256), 0, stream, b,
+                           (const C2<T> *)w, (uint64_t)n_len, (uint64_t)m_len);
     return hipGetLastError();
 }
 
@@ -134,14 +127,6 @@ template <typename T>
 hipError_t bs_scale(C2<T> *z, size_t m_len, double s, hipStream_t stream) {
     hipLaunchKernelGGL((k_bs_scale<T>), grid_1d(m_len), dim3(256), 0, stream, z, (uint64_t)m_len,
                        (T)s);
-    return hipGetLastError();
-}
-
-template <typename T>
-hipError_t bs_digit_swap(const C2<T> *src, C2<T> *dst, size_t n1, size_t m_len,
-                         hipStream_t stream) {
-    hipLaunchKernelGGL((k_bs_digit_swap<T>), grid_1d(m_len), dim3(256), 0, stream, src, dst,
-                       (uint64_t)n1, (uint64_t)m_len);
     return hipGetLastError();
 }
 
@@ -175,7 +160,6 @@ hipError_t bs_post(const C2<T> *c, size_t m_len, C2<T> *out, int64_t out_dist, s
 #define SFFT_BS_INSTANTIATE(T)                                                                  \
     template hipError_t bs_gen_chirp<T>(C2<T> *, C2<T> *, size_t, size_t, hipStream_t);       \
     template hipError_t bs_scale<T>(C2<T> *, size_t, double, hipStream_t);                    \
-    template hipError_t bs_digit_swap<T>(const C2<T> *, C2<T> *, size_t, size_t, hipStream_t); \
     template hipError_t bs_pre<T>(const C2<T> *, int64_t, C2<T> *, size_t, size_t, size_t,    \
                                   const C2<T> *, int, int, int, const C2<T> *, const C2<T> *, \
                                   hipStream_t);                                               \

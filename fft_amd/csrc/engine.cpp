@@ -637,16 +637,22 @@ void Plan::build_bluestein() {
     alloc(&d_chirp_, cn_ * eb);
     alloc(&d_bhat_, bs_m_ * eb);
     table_bytes_ += (cn_ + bs_m_) * eb;
-    alloc(&tmp, bs_m_ * eb);
+    alloc(&tmp, chirp_ ? bs_kernel_work<T>(bs_m_) : bs_m_ * eb);
     struct Free {
         void *p;
         ~Free() { (void)hipFree(p); }
     } free_tmp{tmp};
-    check_hip(bs_gen_chirp<T>((C2<T> *)d_chirp_, (C2<T> *)tmp, cn_, bs_m_, nullptr),
+    check_hip(bs_gen_chirp<T>((C2<T> *)d_chirp_, chirp_ ? nullptr : (C2<T> *)tmp, cn_, bs_m_,
+                              nullptr),
               "chirp generation");
-    bs_inner_->execute(tmp, bs_m_, d_bhat_, bs_m_, 1, 0, nullptr);
-    check_hip(bs_scale<T>((C2<T> *)d_bhat_, bs_m_, 1.0 / (double)bs_m_, nullptr), "chirp scale");
-    if (chirp_) {
+    if (!chirp_) {
+        bs_inner_->execute(tmp, bs_m_, d_bhat_, bs_m_, 1, 0, nullptr);
+        check_hip(bs_scale<T>((C2<T> *)d_bhat_, bs_m_, 1.0 / (double)bs_m_, nullptr),
+                  "chirp scale");
+    } else {
+        check_hip(bs_gen_kernel<T>((C2<T> *)d_bhat_, cn_, bs_m_,
+                                   chirp_cols_ ? (size_t)chirp_cols_->m : 1, tmp, nullptr),
+                  "chirp kernel");
         // stage twiddles of the kernel's radices, taken forwards and backwards
         std::vector<int> rs(chirp_->radices, chirp_->radices + chirp_->nst);
         const std::vector<int> back(rs.rbegin(), rs.rend());
@@ -681,16 +687,10 @@ void Plan::build_bluestein() {
         fill(cs, chirp_twc_);
     }
     if (chirp_cols_) {
-        // the rows' order of the transformed kernel, and their twiddles
-        const size_t n1 = (size_t)chirp_cols_->m, n2 = (size_t)chirp_->m;
         alloc(&d_twist_, bs_m_ * eb);
         table_bytes_ += bs_m_ * eb;
-        check_hip(gen_post_twiddles_full<T>((C2<T> *)d_twist_, n2, bs_m_, nullptr),
+        check_hip(gen_post_twiddles_full<T>((C2<T> *)d_twist_, (size_t)chirp_->m, bs_m_, nullptr),
                   "twiddle generation");
-        check_hip(bs_digit_swap<T>((const C2<T> *)d_bhat_, (C2<T> *)tmp, n1, bs_m_, nullptr),
-                  "chirp order");
-        check_hip(hipMemcpyAsync(d_bhat_, tmp, bs_m_ * eb, hipMemcpyDeviceToDevice, nullptr),
-                  "chirp order");
     }
     check_hip(hipDeviceSynchronize(), "chirp tables");
 }

@@ -73,14 +73,19 @@ template <typename T>
 hipError_t gen_post_twiddles_full(C2<T> *full, size_t n1, size_t N, hipStream_t stream);
 
 // Bluestein (chirp-z) helpers, bluestein.hip.  w: chirp of length N;
-// b: convolution kernel of length M; a / c: per-transform rows of length M.
+// b: convolution kernel of length M (may be null); a / c: per-transform rows of
+// length M.
 template <typename T>
 hipError_t bs_gen_chirp(C2<T> *w, C2<T> *b, size_t n_len, size_t m_len, hipStream_t stream);
 template <typename T>
 hipError_t bs_scale(C2<T> *z, size_t m_len, double s, hipStream_t stream);
-// dst[k1][k2] = src[k1 + n1 k2] over m_len values
+// chirp_table.hip: the transformed convolution kernel over M (primes up to 13),
+// value k1 + n1 k2 at k1 M / n1 + k2, computed in twice the precision of T and
+// rounded once.  work: bs_kernel_work bytes.
 template <typename T>
-hipError_t bs_digit_swap(const C2<T> *src, C2<T> *dst, size_t n1, size_t m_len,
+size_t bs_kernel_work(size_t m_len);
+template <typename T>
+hipError_t bs_gen_kernel(C2<T> *bhat, size_t n_len, size_t m_len, size_t n1, void *work,
                          hipStream_t stream);
 template <typename T>
 hipError_t bs_pre(const C2<T> *in, int64_t in_dist, C2<T> *a, size_t m_len, size_t n_len,
