@@ -183,16 +183,23 @@ int sfft_plan_get_info(sfft_plan plan, sfft_plan_info *info) {
         info->n = p.n();
         info->kind = p.kind();
         info->precision = p.prec();
-        // a chirp-z plan reports the layout of a length-M FFT (run twice, or
-        // once over HBM where both run in one launch)
-        const sfft::Plan &q = p.bluestein() ? *p.bluestein_inner() : p;
-        info->passes = p.bluestein_fused() ? 1 : (int)q.passes().size() * (p.bluestein() ? 2 : 1);
+        info->passes = p.bluestein() ? p.bluestein_passes() : (int)p.passes().size();
         info->chirp_length = p.bluestein_m();
-        const sfft::PassDesc &pd = q.passes()[0].pd;
-        info->nradices = pd.nstages;
-        for (int s = 0; s < pd.nstages && s < 16; ++s) info->radices[s] = pd.st[s].radix;
-        info->threads_per_transform = pd.tpt;
-        info->transforms_per_block = pd.tpw;
+        // a chirp-z plan reports the layout of its first launch: the compiled
+        // chirp kernel, or the first pass of a length-M FFT
+        if (const sfft::ChirpKernel *k = p.chirp_first()) {
+            info->nradices = k->nst;
+            for (int s = 0; s < k->nst && s < 16; ++s) info->radices[s] = k->radices[s];
+            info->threads_per_transform = k->tpt;
+            info->transforms_per_block = k->tpw;
+        } else {
+            const sfft::Plan &q = p.bluestein() ? *p.bluestein_inner() : p;
+            const sfft::PassDesc &pd = q.passes()[0].pd;
+            info->nradices = pd.nstages;
+            for (int s = 0; s < pd.nstages && s < 16; ++s) info->radices[s] = pd.st[s].radix;
+            info->threads_per_transform = pd.tpt;
+            info->transforms_per_block = pd.tpw;
+        }
         info->workspace_bytes = p.workspace_bytes(1, true);
         info->table_bytes = p.table_bytes();
         info->mfma_stages = p.mfma_stages();

@@ -402,7 +402,7 @@ enum : int { kChirpWhole = 0, kChirpRows = 1, kChirpCols = 2 };
 struct ChirpKernel {
     int m, prec;  // convolution, row or column length; 0 F32, 1 F64
     int part;     // kChirpWhole, kChirpRows or kChirpCols
-    int tpw;      // transforms, rows or columns per block
+    int tpt, tpw;  // threads per transform, row or column; these per block
     int nst;
     int radices[kMaxStages];
     // out: the second column pass (kChirpCols)
@@ -433,6 +433,7 @@ struct ChirpReg {
         k.m = M;
         k.prec = sizeof(T) == 8 ? 1 : 0;
         k.part = ROWS ? kChirpRows : kChirpWhole;
+        k.tpt = TPT;
         k.tpw = TPW;
         k.nst = (int)sizeof...(Rs);
         const int rs[] = {Rs...};
@@ -456,6 +457,7 @@ struct ChirpColReg {
         k.m = R0 * R1;
         k.prec = sizeof(T) == 8 ? 1 : 0;
         k.part = kChirpCols;
+        k.tpt = FI::TPT;
         k.tpw = TPW;
         k.nst = 2;
         k.radices[0] = R0;

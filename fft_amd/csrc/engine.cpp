@@ -450,11 +450,13 @@ Plan::Plan(size_t n, int kind, int prec, const PlanHints *h) : n_(n), kind_(kind
         chirp_ = find_chirp(cn_, prec == kF64 ? 1 : 0);
         if (!chirp_) find_chirp_split(cn_, prec == kF64 ? 1 : 0, chirp_cols_, chirp_);
         bs_m_ = !chirp_ ? bs_row_ : (size_t)chirp_->m * (size_t)(chirp_cols_ ? chirp_cols_->m : 1);
-        try {
-            bs_inner_.reset(new Plan(bs_m_, kC2C, prec));
-        } catch (const Error &e) {
-            throw Error(e.code, "size " + std::to_string(n) + " needs a chirp-z length " +
-                                    std::to_string(bs_m_) + ": " + e.what());
+        if (!chirp_) {
+            try {
+                bs_inner_.reset(new Plan(bs_m_, kC2C, prec));
+            } catch (const Error &e) {
+                throw Error(e.code, "size " + std::to_string(n) + " needs a chirp-z length " +
+                                        std::to_string(bs_m_) + ": " + e.what());
+            }
         }
         if (prec == kF64) {
             build_tables<double>();
@@ -938,7 +940,7 @@ void Plan::run(const void *in, size_t in_dist, void *out, size_t out_dist, size_
         run_chirp<T>(in, din, out, dout, batch, inverse, stream, ws);
         return;
     }
-    if (bs_inner_) {
+    if (bluestein()) {
         run_bluestein<T>(in, din, out, dout, batch, inverse, stream, ws);
         return;
     }
@@ -1132,7 +1134,7 @@ template void Plan::run_fixed<double>(const void *, void *, size_t, int, hipStre
 
 size_t Plan::workspace_bytes(size_t batch, bool in_place) const {
     const size_t cb = 2 * real_bytes(prec_);  // one complex value in HBM
-    if (bs_inner_) return 2 * bs_row_ * cb * batch;
+    if (bluestein()) return 2 * bs_row_ * cb * batch;
     if (in_place && passes_.size() > 1) return cn_ * cb * batch;
     return 0;
 }
@@ -1162,7 +1164,7 @@ void Plan::execute(const void *in, size_t in_dist, void *out, size_t out_dist, s
         throw Error(SFFT_ERR_ALIASING, "input and output overlap other than exactly in place");
     if (in_dist < default_in_dist(inverse) || out_dist < default_out_dist(inverse))
         throw Error(SFFT_ERR_INVALID_ARG, "batch distance shorter than one transform");
-    if (bs_inner_ && batch > (0x7fffffffull / bs_row_))
+    if (bluestein() && batch > (0x7fffffffull / bs_row_))
         throw Error(SFFT_ERR_INVALID_ARG, "batch too large");
     const size_t need = workspace_bytes(batch, in_place);
     struct Owned {

@@ -101,7 +101,7 @@ class Plan {
     // in == out (same layout) runs without a workspace: one-pass and chirp-z
     // plans read each transform whole before writing it; two-pass plans run
     // in place through a workspace for the intermediate.
-    bool in_place_direct() const { return bs_inner_ != nullptr || passes_.size() == 1; }
+    bool in_place_direct() const { return bluestein() || passes_.size() == 1; }
     // Device workspace to hand to an execute call of `batch` transforms:
     // chirp-z rows (2 M values per transform, M the smallest 2^a 3^b 5^c
     // convolution length; plans of one launch use none of it, plans of three
@@ -112,11 +112,16 @@ class Plan {
     size_t workspace_used(size_t batch, bool in_place) const;
     // Chirp-z plan: the length has a prime factor the kernels do not plan;
     // the transform runs as a convolution through FFTs of length bluestein_m().
-    bool bluestein() const { return bs_inner_ != nullptr; }
+    bool bluestein() const { return bs_m_ != 0; }
     size_t bluestein_m() const { return bs_m_; }
+    // The plan of the FFTs of the launch sequence; null where compiled chirp
+    // kernels (chirp.h) run the transform: the kernel of its first launch then.
     const Plan *bluestein_inner() const { return bs_inner_.get(); }
-    // ... in one launch, which needs no workspace (chirp.h)
-    bool bluestein_fused() const { return chirp_ && !chirp_cols_; }
+    const ChirpKernel *chirp_first() const { return chirp_cols_ ? chirp_cols_ : chirp_; }
+    // Launches of a chirp-z plan that go through HBM.
+    int bluestein_passes() const {
+        return chirp_cols_ ? 3 : chirp_ ? 1 : 2 * (int)bs_inner_->passes().size();
+    }
 
     // in/out: device pointers; dists in elements of the in/out type
     // (complex for C2C, real/complex for the real kinds).  ws / ws_bytes: a
@@ -181,8 +186,8 @@ class Plan {
     void *d_ptw_full_ = nullptr;  // full four-step table, small plans only
     int ptw_shift_ = 0;
     size_t table_bytes_ = 0;
-    std::unique_ptr<Plan> bs_inner_;
-    size_t bs_m_ = 0;
+    std::unique_ptr<Plan> bs_inner_;  // launch sequence only
+    size_t bs_m_ = 0;                 // 0: not a chirp-z plan
     size_t bs_row_ = 0;  // values per workspace row of the launch sequence
     // the one-launch kernel, or the row kernel of a plan of three launches
     // (then with the column kernels); null: the launch sequence

@@ -91,7 +91,9 @@ typedef struct {
     size_t table_bytes;     /* device twiddle tables held by the plan */
     int mfma_stages;        /* radix-16 stages run as MFMA contractions (16-bit storage) */
     size_t chirp_length;    /* lengths with prime factors > 13: the plan is a chirp-z
-                               convolution through FFTs of this length (0: direct) */
+                               convolution through FFTs of this length (0: direct),
+                               in one launch (passes 1), three (3: columns, rows,
+                               columns) or as separate FFTs (twice their passes) */
     int in_place;           /* 1: in == out (same layout) is allowed (every plan:
                                two-pass lengths run it through the workspace) */
 } sfft_plan_info;
