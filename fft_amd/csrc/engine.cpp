@@ -250,9 +250,28 @@ static const MeasuredSplit kMeasuredSplits16[] = {
 static const MeasuredSplit kMeasuredSplitsF32X[] = {
     {131072, 512}, {524288, 512}, {1048576, 4096},
 };
-// FP64 (2^21 626 -> 522 us, 2^22 716 -> 585, against first passes of 4096):
+// FP64 (2^21 1.17x, 2^22 1.10x; first passes of 1024 and 2048 are as fast, 262
+// and 266 us over both directions of 2^21 x 4, 281 and 268 of 2^22 x 2, but their
+// round trips err 0.9 % and 4 % more):
 static const MeasuredSplit kMeasuredSplitsF64[] = {
-    {2097152, 1024}, {4194304, 2048},
+    {2097152, 4096}, {4194304, 4096},
+};
+
+// Lengths, of every kind, whose split into two compiled column lengths errs more
+// against 64 bits (80 in FP64) than the scored split (forward / round trip:
+// 17496 = 81 x 216 1.09 / 1.21 of 108 x 162, 1638400 1.01 / 1.04, the others
+// 1.005 to 1.03): they take the fastest split that errs no more than the
+// scored one, and is no slower than it for any kind.  Both directions of 128 MB
+// (compiled pair / here / scored): FP64 17496 complex 220 / 250 / 344 us,
+// real 248 / 307 / 433; 1966080 254 / 253 / 340; 1638400, where none but the
+// scored one (1280 x 1280) errs as little, 299 / 398 / 398; FP32 1179648 250 /
+// 300 / 308.
+static const MeasuredSplit kCloserSplits32[] = {
+    {1105920, 1024}, {1179648, 1024}, {2048000, 1280},
+};
+static const MeasuredSplit kCloserSplits64[] = {
+    {14580, 135},    {16200, 135},    {17496, 108},    {1179648, 4096}, {1228800, 4096},
+    {1310720, 1280}, {1572864, 3072}, {1638400, 1280}, {1966080, 3840},
 };
 
 template <size_t K>
@@ -548,12 +567,15 @@ Plan::Plan(size_t n, int kind, int prec, const PlanHints *h) : n_(n), kind_(kind
         // variant choice, keep the table's split: a plan and its
         // runtime-planned variant compute the same factorisation)
         const bool free_split = !h || (h->split == 0 && h->radices.empty() && !h->tpw);
-        size_t table_n1 = 0;
-        if (free_split && prec == kF32)
+        size_t table_n1 = !free_split     ? 0
+                          : prec == kF32 ? lookup_split(kCloserSplits32, cn_)
+                          : prec == kF64 ? lookup_split(kCloserSplits64, cn_)
+                                         : 0;
+        if (!table_n1 && free_split && prec == kF32)
             table_n1 = kind == kC2C   ? lookup_split(kMeasuredSplits, cn_)
                        : kind == kR2C ? lookup_split(kMeasuredRealSplits, cn_)
                                       : 0;
-        else if (free_split && kind == kC2C)
+        else if (!table_n1 && free_split && kind == kC2C)
             table_n1 = stored_16(prec)  ? lookup_split(kMeasuredSplits16, cn_)
                        : prec == kF32X ? lookup_split(kMeasuredSplitsF32X, cn_)
                        : prec == kF64  ? lookup_split(kMeasuredSplitsF64, cn_)
@@ -562,9 +584,8 @@ Plan::Plan(size_t n, int kind, int prec, const PlanHints *h) : n_(n), kind_(kind
         // FP64, 128 MB batches, against the scored split with its runtime-planned
         // passes: 331776 172 -> 110 us, 1000000 188 -> 144, FP64 708588
         // 180 -> 140, R2C 839808 270 -> 180), else any
-        const bool prefer = free_split;
         if (table_n1) search(table_n1, compiled_split);
-        if (!best_n1 && (compiled_split || prefer)) search(0, true);
+        if (!best_n1 && (compiled_split || free_split)) search(0, true);
         if (!best_n1 && !compiled_split) search(0, false);
         if (!best_n1 && !ok)
             throw Error(SFFT_ERR_UNSUPPORTED_SIZE,
