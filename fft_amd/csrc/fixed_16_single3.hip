@@ -1,13 +1,20 @@
 // fixed_16_single3.hip -- compile-time plans with 16-bit storage
 // (float LDS and arithmetic), single pass: part 4 of 8 of the fast lengths
 // other than powers of two.
-// Radices are those the runtime planner's cost model chooses at 16 elements a
-// thread, so that bits and every other use of the plan stay as they were;
-// about 256 threads a block; one group per block (the persistent form of these
-// kernels had lost).  Bound by HBM.  Listed where faster over both directions
-// with neither 3 % slower, batches of 128 MB:
-// median 1.52x over the runtime-planned pass, up to 3.9x above 8192; 200, 2500
-// and 15000 are no faster.
+// Radices are those the runtime planner's cost model chooses within the 512
+// threads of a 16-bit block, so that bits and strided calls (which run the
+// runtime-planned pass) stay as they were: the radices of 1024 threads made
+// strided calls of 14 lengths 1.1 to 2.1x slower (both directions of 128 MB:
+// 6912 267 -> 562 us, 13122 588 -> 965).  Six lengths take those all the same,
+// because batches gain and strided calls do not lose (batches / strided, 512 ->
+// 1024: 6561 308 / 496 -> 165 / 475, 8100 224 / 573 -> 188 / 502, 11250 243 / 646
+// -> 222 / 570, 13500 249 / 569 -> 236 / 570, 14400 181 / 518 -> 174 / 521, 15360
+// 182 / 478 -> 172 / 483).  Threads are free (the bits do not depend on them):
+// about 256 a block, from 4860 on the multiple of the butterflies that idles least;
+// one group per block (the persistent form of these kernels had lost).  Bound by
+// HBM.  Listed where faster over both directions with neither 3 % slower, batches
+// of 128 MB: median 1.5x over the runtime-planned pass, up to 3.5x above 7500;
+// 200, 2500 and 15000 are no faster.
 #include "fixed.h"
 
 namespace sfft {
@@ -31,10 +38,10 @@ struct One {
     const FixedC2C<E, 4608, 384, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 12, 12, 2> c4608;
     const FixedC2C<E, 5760, 384, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 15, 8, 3> c5760;
     const FixedC2C<E, 6561, 729, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 9, 9, 9, 9> c6561;
-    const FixedC2C<E, 8000, 800, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 10, 10, 10, 8> c8000;
-    const FixedC2C<E, 9720, 810, 1, Sched<kNoPrefetch, 0, 0, 0, kLdsPadShift>, 0, 15, 6, 6, 6, 3> c9720;
+    const FixedC2C<E, 8000, 800, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 10, 10, 5> c8000;
+    const FixedC2C<E, 9720, 648, 1, Sched<kNoPrefetch, 0, 0, 0, kLdsPadShift>, 0, 15, 9, 9, 8> c9720;
     const FixedC2C<E, 11520, 768, 1, Sched<kNoPrefetch, 0, 0, 0, kLdsPadShift>, 0, 16, 16, 15, 3> c11520;
-    const FixedC2C<E, 13122, 875, 1, Sched<kNoPrefetch, 0, 0, 0, kLdsPadShift>, 0, 3, 3, 3, 3, 3, 3, 3, 3, 2> c13122;
+    const FixedC2C<E, 13122, 729, 1, Sched<kNoPrefetch, 0, 0, 0, kLdsPadShift>, 0, 9, 9, 9, 9, 2> c13122;
 };
 const One<StoreF16> f16;
 const One<StoreBF16> bf16;

@@ -1,13 +1,20 @@
 // fixed_16_single5.hip -- compile-time plans with 16-bit storage
 // (float LDS and arithmetic), single pass: part 6 of 8 of the fast lengths
 // other than powers of two.
-// Radices are those the runtime planner's cost model chooses at 16 elements a
-// thread, so that bits and every other use of the plan stay as they were;
-// about 256 threads a block; one group per block (the persistent form of these
-// kernels had lost).  Bound by HBM.  Listed where faster over both directions
-// with neither 3 % slower, batches of 128 MB:
-// median 1.52x over the runtime-planned pass, up to 3.9x above 8192; 200, 2500
-// and 15000 are no faster.
+// Radices are those the runtime planner's cost model chooses within the 512
+// threads of a 16-bit block, so that bits and strided calls (which run the
+// runtime-planned pass) stay as they were: the radices of 1024 threads made
+// strided calls of 14 lengths 1.1 to 2.1x slower (both directions of 128 MB:
+// 6912 267 -> 562 us, 13122 588 -> 965).  Six lengths take those all the same,
+// because batches gain and strided calls do not lose (batches / strided, 512 ->
+// 1024: 6561 308 / 496 -> 165 / 475, 8100 224 / 573 -> 188 / 502, 11250 243 / 646
+// -> 222 / 570, 13500 249 / 569 -> 236 / 570, 14400 181 / 518 -> 174 / 521, 15360
+// 182 / 478 -> 172 / 483).  Threads are free (the bits do not depend on them):
+// about 256 a block, from 4860 on the multiple of the butterflies that idles least;
+// one group per block (the persistent form of these kernels had lost).  Bound by
+// HBM.  Listed where faster over both directions with neither 3 % slower, batches
+// of 128 MB: median 1.5x over the runtime-planned pass, up to 3.5x above 7500;
+// 200, 2500 and 15000 are no faster.
 #include "fixed.h"
 
 namespace sfft {
@@ -28,13 +35,13 @@ struct One {
     const FixedC2C<E, 2560, 256, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 16, 10> c2560;
     const FixedC2C<E, 3200, 200, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 25, 16, 8> c3200;
     const FixedC2C<E, 3888, 432, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 12, 9, 6, 6> c3888;
-    const FixedC2C<E, 4860, 540, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 10, 9, 9, 6> c4860;
+    const FixedC2C<E, 4860, 405, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 15, 6, 6, 3, 3> c4860;
     const FixedC2C<E, 6000, 400, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 25, 16, 15> c6000;
-    const FixedC2C<E, 6912, 576, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 12, 6, 6> c6912;
-    const FixedC2C<E, 8640, 720, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 12, 12, 12, 5> c8640;
+    const FixedC2C<E, 6912, 432, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 16, 3, 3, 3> c6912;
+    const FixedC2C<E, 8640, 720, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 15, 6, 6> c8640;
     const FixedC2C<E, 10125, 675, 1, Sched<kNoPrefetch, 0, 0, 0, kLdsPadShift>, 0, 15, 15, 15, 3> c10125;
-    const FixedC2C<E, 12000, 800, 1, Sched<kNoPrefetch, 0, 0, 0, kLdsPadShift>, 0, 25, 16, 15, 2> c12000;
-    const FixedC2C<E, 13824, 922, 1, Sched<kNoPrefetch, 0, 0, 0, kLdsPadShift>, 0, 16, 16, 3, 3, 3, 2> c13824;
+    const FixedC2C<E, 12000, 800, 1, Sched<kNoPrefetch, 0, 0, 0, kLdsPadShift>, 0, 16, 15, 10, 5> c12000;
+    const FixedC2C<E, 13824, 864, 1, Sched<kNoPrefetch, 0, 0, 0, kLdsPadShift>, 0, 16, 16, 9, 6> c13824;
 };
 const One<StoreF16> f16;
 const One<StoreBF16> bf16;

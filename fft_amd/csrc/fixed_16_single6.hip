@@ -1,13 +1,20 @@
 // fixed_16_single6.hip -- compile-time plans with 16-bit storage
 // (float LDS and arithmetic), single pass: part 7 of 8 of the fast lengths
 // other than powers of two.
-// Radices are those the runtime planner's cost model chooses at 16 elements a
-// thread, so that bits and every other use of the plan stay as they were;
-// about 256 threads a block; one group per block (the persistent form of these
-// kernels had lost).  Bound by HBM.  Listed where faster over both directions
-// with neither 3 % slower, batches of 128 MB:
-// median 1.52x over the runtime-planned pass, up to 3.9x above 8192; 200, 2500
-// and 15000 are no faster.
+// Radices are those the runtime planner's cost model chooses within the 512
+// threads of a 16-bit block, so that bits and strided calls (which run the
+// runtime-planned pass) stay as they were: the radices of 1024 threads made
+// strided calls of 14 lengths 1.1 to 2.1x slower (both directions of 128 MB:
+// 6912 267 -> 562 us, 13122 588 -> 965).  Six lengths take those all the same,
+// because batches gain and strided calls do not lose (batches / strided, 512 ->
+// 1024: 6561 308 / 496 -> 165 / 475, 8100 224 / 573 -> 188 / 502, 11250 243 / 646
+// -> 222 / 570, 13500 249 / 569 -> 236 / 570, 14400 181 / 518 -> 174 / 521, 15360
+// 182 / 478 -> 172 / 483).  Threads are free (the bits do not depend on them):
+// about 256 a block, from 4860 on the multiple of the butterflies that idles least;
+// one group per block (the persistent form of these kernels had lost).  Bound by
+// HBM.  Listed where faster over both directions with neither 3 % slower, batches
+// of 128 MB: median 1.5x over the runtime-planned pass, up to 3.5x above 7500;
+// 200, 2500 and 15000 are no faster.
 #include "fixed.h"
 
 namespace sfft {
@@ -32,8 +39,8 @@ struct One {
     const FixedC2C<E, 6075, 405, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 15, 15, 3, 3, 3> c6075;
     const FixedC2C<E, 7200, 480, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 15, 15, 2> c7200;
     const FixedC2C<E, 8748, 972, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 12, 9, 9, 9> c8748;
-    const FixedC2C<E, 10240, 683, 1, Sched<kNoPrefetch, 0, 0, 0, kLdsPadShift>, 0, 16, 16, 8, 5> c10240;
-    const FixedC2C<E, 12150, 1013, 1, Sched<kNoPrefetch, 0, 0, 0, kLdsPadShift>, 0, 15, 15, 6, 3, 3> c12150;
+    const FixedC2C<E, 10240, 640, 1, Sched<kNoPrefetch, 0, 0, 0, kLdsPadShift>, 0, 16, 16, 10, 4> c10240;
+    const FixedC2C<E, 12150, 810, 1, Sched<kNoPrefetch, 0, 0, 0, kLdsPadShift>, 0, 15, 10, 9, 9> c12150;
     const FixedC2C<E, 14400, 960, 1, Sched<kNoPrefetch, 0, 0, 0, kLdsPadShift>, 0, 16, 15, 15, 4> c14400;
 };
 const One<StoreF16> f16;
