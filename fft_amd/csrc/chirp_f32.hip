@@ -7,11 +7,12 @@
 // ps per element of M against 4.9 at 1024 and 2048, at 8 to 16 transforms
 // resident per CU).  Two transforms per thread, which halves the table loads,
 // measured 0.62-0.98x: half the resident waves.
-// 1024 and 2048 take eight elements a thread and one more stage, which
+// 1024, 2048 and 4096 take eight elements a thread and one more stage, which
 // halves a wave's registers and LDS (twice the waves).  Both directions, sixteen
-// / eight: 509 x 8192 68.2 / 64.8 us, 1009 x 4096 73.4 / 68.2, x 20000 376 / 321, one
-// transform of 1009 17.1 / 11.3.  4096 would be 3 % faster too, but its inverse
-// error was 3.6e-7 where separate launches had 3.5e-7 (n = 1999).
+// / eight: 509 x 8192 68.2 / 64.8 us, 1009 x 4096 73.4 / 68.2, x 20000 376 / 321,
+// 1999 x 2048 74.4 / 70.6, 2029 x 20000 856 / 765, and one transform of 1009 17.1 /
+// 11.3, of 1999 18.0 / 14.2.  The shorter radices err less too (round trips of
+// the lengths that 4096 serves: 0.774 / 0.739 of the separate launches' error).
 #include "chirp.h"
 
 namespace sfft {
@@ -30,6 +31,6 @@ const ChirpReg<float, false, 1024, 128, 2, 4, 8, 4, 4, 8> c1024;
 const ChirpReg<float, false, 1536, 96, 2, 3, 16, 6, 16> c1536;
 const ChirpReg<float, false, 2048, 256, 1, 4, 8, 8, 4, 8> c2048;
 const ChirpReg<float, false, 3072, 256, 1, 4, 16, 16, 12> c3072;
-const ChirpReg<float, false, 4096, 256, 1, 4, 16, 16, 16> c4096;
+const ChirpReg<float, false, 4096, 512, 1, 4, 8, 8, 8, 8> c4096;
 }  // namespace
 }  // namespace sfft
