@@ -18,7 +18,7 @@ UnevenBatch::UnevenBatch(const sfft_batch_item *items, size_t count, int prec)
         // launch sequence after the persistent launch, in the same graph,
         // through one workspace sized for the largest of them
         if (plans_.back()->bluestein())
-            ws_bytes_ = std::max(ws_bytes_, plans_.back()->workspace_bytes(it.count, false));
+            ws_bytes_ = std::max(ws_bytes_, plans_.back()->workspace_used(it.count, false));
     }
 
     const size_t lds_cap = device_info().lds_bytes;

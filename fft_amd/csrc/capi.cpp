@@ -238,8 +238,11 @@ int sfft_execute_workspace(sfft_plan plan, const void *in, void *out, size_t bat
             return fail(SFFT_ERR_INVALID_ARG, "direction must be SFFT_FORWARD or SFFT_INVERSE");
         const sfft::Plan &p = *plan->plan;
         const bool in_place = in != nullptr && in == out;
-        if (p.workspace_bytes(batch, in_place) && !workspace)
-            return fail(SFFT_ERR_INVALID_ARG, "this call needs a workspace");
+        const size_t need = p.workspace_bytes(batch, in_place);
+        if (need && !workspace) return fail(SFFT_ERR_INVALID_ARG, "this call needs a workspace");
+        if (workspace_bytes < need)
+            return fail(SFFT_ERR_INVALID_ARG, "workspace of " + std::to_string(workspace_bytes) +
+                                                  " bytes, the call needs " + std::to_string(need));
         p.execute(in, p.default_in_dist(direction), out, p.default_out_dist(direction), batch,
                   direction, (hipStream_t)stream, workspace, workspace_bytes);
         return SFFT_OK;

@@ -1187,7 +1187,7 @@ void Plan::execute(const void *in, size_t in_dist, void *out, size_t out_dist, s
         throw Error(SFFT_ERR_INVALID_ARG, "batch distance shorter than one transform");
     if (bluestein() && batch > (0x7fffffffull / bs_row_))
         throw Error(SFFT_ERR_INVALID_ARG, "batch too large");
-    const size_t need = workspace_bytes(batch, in_place);
+    const size_t need = workspace_bytes(batch, in_place), use = workspace_used(batch, in_place);
     struct Owned {
         void *p = nullptr;
         hipStream_t s = nullptr;
@@ -1196,13 +1196,14 @@ void Plan::execute(const void *in, size_t in_dist, void *out, size_t out_dist, s
         }
     } owned;
     if (need && ws) {
-        if (ws_bytes < need)
+        if (ws_bytes < use)
             throw Error(SFFT_ERR_INVALID_ARG, "workspace of " + std::to_string(ws_bytes) +
-                                                  " bytes, the call needs " + std::to_string(need));
+                                                  " bytes, the call uses " + std::to_string(use));
         const uintptr_t w0 = (uintptr_t)ws;
-        if ((w0 < i0 + in_len && i0 < w0 + need) || (w0 < o0 + out_len && o0 < w0 + need))
+        const size_t len = std::min(ws_bytes, need);
+        if ((w0 < i0 + in_len && i0 < w0 + len) || (w0 < o0 + out_len && o0 < w0 + len))
             throw Error(SFFT_ERR_ALIASING, "workspace overlaps the input or the output");
-    } else if (const size_t use = workspace_used(batch, in_place)) {
+    } else if (use) {
         if (hipMallocAsync(&owned.p, use, stream) != hipSuccess) {
             (void)hipGetLastError();
             owned.p = nullptr;

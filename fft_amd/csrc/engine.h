@@ -102,13 +102,13 @@ class Plan {
     // plans read each transform whole before writing it; two-pass plans run
     // in place through a workspace for the intermediate.
     bool in_place_direct() const { return bluestein() || passes_.size() == 1; }
-    // Device workspace to hand to an execute call of `batch` transforms:
-    // chirp-z rows (2 M values per transform, M the smallest 2^a 3^b 5^c
-    // convolution length; plans of one launch use none of it, plans of three
-    // about half) or, in place on a two-pass length, the intermediate (cn values per
-    // transform); 0 if none.
+    // Device workspace that the C ABI asks a caller for (an upper bound for every
+    // launch plan of the length): chirp-z rows (2 M values per transform, M the
+    // smallest 2^a 3^b 5^c convolution length) or, in place on a two-pass length,
+    // the intermediate (cn values per transform); 0 if none.
     size_t workspace_bytes(size_t batch, bool in_place) const;
-    // What such a call uses of it.
+    // What the call uses of it, which is what the library itself allocates or
+    // reserves: chirp-z plans of one launch none, of three M values per transform.
     size_t workspace_used(size_t batch, bool in_place) const;
     // Chirp-z plan: the length has a prime factor the kernels do not plan;
     // the transform runs as a convolution through FFTs of length bluestein_m().
@@ -125,7 +125,7 @@ class Plan {
 
     // in/out: device pointers; dists in elements of the in/out type
     // (complex for C2C, real/complex for the real kinds).  ws / ws_bytes: a
-    // caller's device workspace of at least workspace_bytes(batch, in == out)
+    // caller's device workspace of at least workspace_used(batch, in == out)
     // bytes; without one, a needed workspace is allocated stream-ordered
     // (hipMallocAsync) and freed after the call.
     void execute(const void *in, size_t in_dist, void *out, size_t out_dist, size_t batch,

@@ -60,7 +60,7 @@ extern "C" int sfft_execute_noalloc(sfft_plan plan, const void *in, void *out, s
                               "direction must be SFFT_FORWARD or SFFT_INVERSE");
         const sfft::Plan &p = *plan->plan;
         const bool in_place = in != nullptr && in == out;
-        const size_t need = p.workspace_bytes(batch, in_place);
+        const size_t need = p.workspace_used(batch, in_place);
         if (need > kScratchBytes)
             throw sfft::Error(SFFT_ERR_BUDGET,
                               "sfft_execute_noalloc: this call needs " + std::to_string(need) +

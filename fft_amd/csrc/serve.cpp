@@ -171,7 +171,7 @@ class Server {
             r->plan = get_plan(rq.n, rq.kind, cfg_.precision);
             r->in_bytes = r->plan->in_bytes(rq.batch, rq.direction);
             r->out_bytes = r->plan->out_bytes(rq.batch, rq.direction);
-            r->ws_bytes = r->plan->workspace_bytes(rq.batch, false);
+            r->ws_bytes = r->plan->workspace_used(rq.batch, false);
             const size_t need =
                 align256(r->in_bytes) + align256(r->out_bytes) + align256(r->ws_bytes);
             if (need > pool_->size())

@@ -87,7 +87,8 @@ typedef struct {
     int radices[16];
     int threads_per_transform, transforms_per_block;
     size_t workspace_bytes; /* device workspace per transform of an in-place call
-                               (chirp-z lengths: every call); 0: none */
+                               (chirp-z lengths: every call), as
+                               sfft_plan_workspace_size has it; 0: none */
     size_t table_bytes;     /* device twiddle tables held by the plan */
     int mfma_stages;        /* radix-16 stages run as MFMA contractions (16-bit storage) */
     size_t chirp_length;    /* lengths with prime factors > 13: the plan is a chirp-z
@@ -189,13 +190,16 @@ int sfft_tune_clear(void);
  * in == out transforms in place (the reference accepts any iterator pair,
  * signalsmith-fft.h:55-67, but corrupts in place); other overlaps return
  * SFFT_ERR_ALIASING.  Chirp-z lengths, and two-pass lengths in place, need
- * a device workspace (sfft_plan_workspace_size): sfft_execute allocates it
- * stream-ordered (hipMallocAsync, released after the call). */
+ * a device workspace (sfft_plan_workspace_size): sfft_execute allocates what
+ * it uses stream-ordered (hipMallocAsync, released after the call). */
 int sfft_execute(sfft_plan plan, const void *in, void *out, size_t batch, int direction,
                  void *stream);
 
-/* Bytes of device workspace an execute call of `batch` transforms needs
- * (in_place: in == out); 0 if none. */
+/* Bytes of device workspace to hand to an execute call of `batch` transforms
+ * (in_place: in == out); 0 if none.  For chirp-z lengths an upper bound that
+ * depends on the length alone: two rows of the smallest 2^a 3^b 5^c length
+ * >= 2n - 1 a transform, of which plans of one launch use none and plans of
+ * three launches about half. */
 int sfft_plan_workspace_size(sfft_plan plan, size_t batch, int in_place, size_t *bytes);
 /* sfft_execute with a caller-owned device workspace of at least
  * sfft_plan_workspace_size bytes (may be NULL when that is 0): the call
@@ -209,7 +213,7 @@ int sfft_execute_workspace(sfft_plan plan, const void *in, void *out, size_t bat
  * tight serving loops, harnesses that forbid hipMalloc).  The workspace a
  * call needs (chirp-z lengths; two-pass lengths in place) comes from a
  * library-owned static device array of SFFT_NOALLOC_SCRATCH_BYTES per GPU,
- * held until the process ends; a call needing more returns SFFT_ERR_BUDGET.
+ * held until the process ends; a call that uses more returns SFFT_ERR_BUDGET.
  * Every call on a GPU shares that GPU's array: calls that overlap on one GPU
  * (other streams, other threads) race. */
 #define SFFT_NOALLOC_SCRATCH_BYTES ((size_t)64 << 20)
