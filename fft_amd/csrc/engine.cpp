@@ -420,14 +420,16 @@ static void use_fixed_columns(PassPlan &pp, size_t n, int prec, int mode, bool r
     }
 }
 
-// A wider tile with the radices the pass has taken (so the same bits).
-static void use_wide_columns(PassPlan &pp, size_t n, int prec, int mode) {
-    const FixedKernel *fk = find_fixed((int)n, prec, 3, -1);
+// A wider (registry kind 3) or narrower (4) tile with the radices the pass has
+// taken (so the same bits).
+static void use_tile(PassPlan &pp, size_t n, int prec, int mode, int reg,
+                     const FixedKernel *&tile, unsigned &grid) {
+    const FixedKernel *fk = find_fixed((int)n, prec, reg, -1);
     if (!fk || fk->nst != pp.pd.nstages) return;
     for (int s = 0; s < fk->nst; ++s)
         if (fk->radices[s] != pp.pd.st[s].radix) return;
-    pp.wide = fk;
-    pp.wide_grid = (unsigned)(fk->blocks_per_cu(mode) * device_info().cu_count);
+    tile = fk;
+    grid = (unsigned)(fk->blocks_per_cu(mode) * device_info().cu_count);
 }
 
 // 16-bit storage: run the pass' radix-16 stages on MFMA when every wave of
@@ -623,8 +625,9 @@ Plan::Plan(size_t n, int kind, int prec, const PlanHints *h) : n_(n), kind_(kind
         if (!(h && (h->tpw || h->fixed_variant == -2 || (stored_16(prec) && h->mfma == 1)))) {
             use_fixed_columns(p1, n1, prec, kModeColRow, kind != kC2C);
             use_fixed_columns(p2, n2, prec, kModeColCol, kind != kC2C);
-            use_wide_columns(p1, n1, prec, kModeColRow);
-            use_wide_columns(p2, n2, prec, kModeColCol);
+            use_tile(p1, n1, prec, kModeColRow, 3, p1.wide, p1.wide_grid);
+            use_tile(p2, n2, prec, kModeColCol, 3, p2.wide, p2.wide_grid);
+            use_tile(p1, n1, prec, kModeColRow, 4, p1.narrow, p1.narrow_grid);
         }
         passes_.push_back(p1);
         passes_.push_back(p2);
@@ -1001,6 +1004,13 @@ void Plan::run_passes(const void *in, int64_t din, void *out, int64_t dout, size
             pp.slots_per_transform % pp.wide->tpw == 0 &&
             slots / (size_t)pp.wide->tpw >= (size_t)device_info().cu_count) {
             run_fixed_columns<T>(p, *pp.wide, cm, pp.wide_grid, src, dsrc, dst, ddst, batch,
+                                 inverse, stream);
+            continue;
+        }
+        if (cm == kModeColRow && pp.narrow && pp.fixed &&
+            slots / (size_t)pp.fixed->row_tpw * (size_t)pp.narrow->cus_per_tile <
+                (size_t)device_info().cu_count) {
+            run_fixed_columns<T>(p, *pp.narrow, cm, pp.narrow_grid, src, dsrc, dst, ddst, batch,
                                  inverse, stream);
             continue;
         }

@@ -72,6 +72,9 @@ struct PassPlan {
     // every CU a tile
     const FixedKernel *wide = nullptr;
     unsigned wide_grid = 0;
+    // narrower tiles of a plain first pass (same bits), for launches of few
+    const FixedKernel *narrow = nullptr;
+    unsigned narrow_grid = 0;
 };
 
 // Overrides the planner's choice (autotuner candidates).

@@ -877,9 +877,11 @@ struct FixedKernel {
     int real;       // 0: C2C kernel; 1: real pair (R2C forward + C2R inverse);
                     // 2: column passes of two-pass plans (kModeColRow, kModeColCol)
                     // 3: the same in wider tiles, for launches that fill the device
+                    // 4: kModeColRow in narrower tiles, for launches of few
     bool paired;    // 2: with the paired modes of real transforms
     int tpt, tpw;
-    int row_tpw, col_tpw;  // 2, 3: columns per block in kModeColRow, kModeColCol
+    int row_tpw, col_tpw;  // 2 to 4: columns per block in kModeColRow, kModeColCol
+    int cus_per_tile;  // 4: for launches of less than a (wide) tile per so many CUs
     int nst;
     int radices[kMaxStages];
     size_t lds_bytes;
@@ -1031,6 +1033,28 @@ struct FixedColOf {
 template <typename T, int N, int TPT, int TPW, int WR, int WC, class SCH, int... Rs>
 using FixedCol =
     FixedColOf<T, N, TPT, TPW, WR, WC, SCH, 0, std::is_arithmetic<T>::value, 2, Rs...>;
+// Registers the plain first pass in a narrower tile (registry kind 4), for
+// launches of less than a tile of the ordinary width per CUS compute units.
+template <typename T, int N, int TPT, int TPW, int CUS, class SCH, int... Rs>
+struct FixedRowNarrow {
+    using F = Fixed<T, N, TPT, TPW, kModeColRow, SCH, Rs...>;
+    FixedRowNarrow() {
+        FixedKernel k{};
+        k.n = N;
+        k.prec = FixedElem<T>::prec;
+        k.real = 4;
+        k.tpt = TPT;
+        k.tpw = k.row_tpw = TPW;
+        k.cus_per_tile = CUS;
+        fixed_fill_radices<Rs...>(k);
+        k.lds_bytes = F::LDS_BYTES;
+        k.launch = [](const void *args, int, unsigned grid, hipStream_t s) {
+            return fixed_launch_one<F>(args, grid, s);
+        };
+        k.blocks_per_cu = [](int) { return fixed_occupancy<F>(); };
+        register_fixed(k);
+    }
+};
 template <typename T, int N, int TPT, int TPW, class SCH, int... Rs>
 using FixedColWide = FixedColOf<T, N, TPT, TPW, TPW, TPW, SCH, 0, false, 3, Rs...>;
 

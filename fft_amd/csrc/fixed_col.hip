@@ -7,6 +7,12 @@
 // the first pass, whose input comes from HBM (128: 64 columns 103 us, 32 112, 16
 // 123), more blocks in the second, which reads what the last-level cache still
 // holds (512: 8 columns 81 us, 16 89; 2048: 4 columns 104, 8 122).
+// Such a wide first pass leaves CUs idle where a launch has few tiles.  Below a
+// tile per CU 128 and 144 take half the width, and 625 below a tile per two
+// (FixedRowNarrow<..., columns, CUs per tile, ...>; both directions, wide / narrow:
+// 20736 x 21 24.9 / 20.0 us, x 102 45.0 / 40.9, 90000 x 26 51.8 / 38.3, 16000 x 64
+// 32.3 / 29.3, x 131 48.0 / 46.5; 625: 78125 x 14 37.8 / 33.2, but x 26 44.0 /
+// 59.3).  81 gains and loses 4 % and keeps the wide one.
 // FP32 and FP64 first passes read their input non-temporally (Sched NT 1;
 // 2^19 x 64 and 2^18 x 128 +13-15 %, 1024 and 2048 +3-6 %); non-temporal output
 // stores of the second pass slowed the lengths whose output is read back (the
@@ -16,6 +22,7 @@
 namespace sfft {
 namespace {
 const FixedCol<float, 128, 8, 32, 64, 32, Sched<0, 0, 0, 0, kLdsPadShift, 1>, 16, 8> col128;
+const FixedRowNarrow<float, 128, 8, 32, 1, Sched<0, 0, 0, 0, kLdsPadShift, 1>, 16, 8> row128;
 const FixedCol<float, 256, 16, 32, 32, 32, Sched<0, 0, 0, 0, kLdsPadShift, 1>, 16, 16> col256;
 const FixedCol<float, 512, 32, 16, 16, 8, Sched<0, 0, 0, 0, kLdsPadShift, 1>, 16, 16, 2> col512;
 const FixedCol<float, 1024, 64, 8, 8, 8, Sched<0, 0, 0, 0, kLdsPadShift, 1>, 16, 16, 4> col1024;

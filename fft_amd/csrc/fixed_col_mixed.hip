@@ -30,6 +30,7 @@ const FixedCol<float, 300, 20, 32, 16, 16, Sched<0, 0, 0, 0, kLdsNoPad, 1>, 15, 
 const FixedCol<float, 270, 23, 32, 32, 32, Sched<0, 0, 0, 0, kLdsNoPad, 1>, 15, 6, 3> col270;
 const FixedCol<float, 288, 24, 32, 32, 16, Sched<0, 0, 0, 0, kLdsNoPad, 1>, 12, 12, 2> col288;
 const FixedCol<float, 625, 25, 8, 16, 8, Sched<0, 0, 0, 0, kLdsNoPad, 1>, 25, 25> col625;
+const FixedRowNarrow<float, 625, 25, 8, 2, Sched<0, 0, 0, 0, kLdsNoPad, 1>, 25, 25> row625;
 const FixedCol<float, 225, 15, 32, 32, 32, Sched<0, 0, 0, 0, kLdsNoPad, 1>, 15, 15> col225;
 const FixedCol<float, 240, 16, 32, 32, 32, Sched<0, 0, 0, 0, kLdsNoPad, 1>, 16, 15> col240;
 const FixedCol<float, 200, 13, 32, 32, 32, Sched<0, 0, 0, 0, kLdsNoPad, 1>, 25, 8> col200;
@@ -49,6 +50,7 @@ const FixedCol<float, 540, 45, 16, 16, 16, Sched<0, 0, 0, 0, kLdsNoPad, 1>, 15, 
 const FixedCol<float, 125, 5, 64, 64, 64, Sched<0, 0, 0, 0, kLdsNoPad, 1>, 25, 5> col125;
 const FixedCol<float, 729, 81, 8, 8, 8, Sched<0, 0, 0, 0, kLdsNoPad, 1>, 9, 9, 9> col729;
 const FixedCol<float, 144, 12, 32, 64, 32, Sched<0, 0, 0, 0, kLdsNoPad, 1>, 12, 12> col144;
+const FixedRowNarrow<float, 144, 12, 32, 1, Sched<0, 0, 0, 0, kLdsNoPad, 1>, 12, 12> row144;
 const FixedCol<float, 135, 15, 32, 32, 32, Sched<0, 0, 0, 0, kLdsNoPad, 1>, 15, 9> col135;
 const FixedCol<float, 81, 9, 32, 64, 32, Sched<0, 0, 0, 0, kLdsNoPad, 1>, 9, 9> col81;
 }  // namespace
