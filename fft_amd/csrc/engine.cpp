@@ -971,6 +971,17 @@ void Plan::run(const void *in, size_t in_dist, void *out, size_t out_dist, size_
     run_passes<T>(in, din, out, dout, batch, inverse, stream, ws);
 }
 
+// Column launches whose data stays in the XCDs' L2 caches (8 x 4 MB) between the
+// passes: each XCD then takes whole transforms (fixed.h), so a launch needs some
+// for each.  Time against tiles dealt to the XCDs in turn, 140 two-pass lengths of
+// every kind (geometric mean): with 16 or more transforms 0.87 at 12 to 18 MB,
+// 0.92 to 26 MB, 0.94 (complex FP32 and FP64) at 32 MB, 1.00 at 40; with 8 to 15
+// 0.93 to 14 MB, then 0.96 to 1.02 and up to 1.18 at single lengths; below 8 1.00.
+static bool near_launch(size_t batch, size_t bytes) {
+    return batch >= 2 * kXcds ? bytes <= (size_t)34 << 20
+                              : batch >= kXcds && bytes <= (size_t)14 << 20;
+}
+
 // Columns per block of a column kernel in a mode.
 static int column_tile(const FixedKernel &fk, int mode) {
     return mode == kModeColRow || mode == kModeColRowRot   ? fk.row_tpw
@@ -1139,6 +1150,7 @@ void Plan::run_fixed_columns(size_t p, const FixedKernel &fk, int mode, unsigned
         a.real_tw = (const C2<T> *)d_real_tw_;
         a.half_shift = kind_ == kR2CHalf;
         a.rot = (const C2<T> *)d_rot_;
+        a.near = near_launch(cb, cb * cn_ * eb);
         a.in_bs = (int32_t)dsrc;
         a.in_ss = (int32_t)pp.in_slot_stride;
         a.in_es = (int32_t)pp.in_elem_stride;

@@ -52,6 +52,7 @@ struct FixedArgs {
     const C2<T> *ptw_fine, *ptw_coarse;
     const C2<T> *ptw_full;  // or null: W_N^{c e} at c N + e (N: this pass' length)
     FastDiv tiles;  // paired column modes: tiles per transform
+    uint32_t near;  // column modes: the launch's data fits the L2 caches
 };
 
 // Paired column modes.  Bin m = c + S e of a two-pass real transform (column c
@@ -806,16 +807,18 @@ struct Fixed {
             const auto odd_pitch = [](int32_t es) {
                 return es != 1 && (((uint32_t)es * DB) & 127u) != 0;
             };
-            const bool share = PAIR || NARROW || odd_pitch(a.in_es) || odd_pitch(a.out_es);
+            const bool share =
+                PAIR || NARROW || a.near || odd_pitch(a.in_es) || odd_pitch(a.out_es);
             // (One tile per block: windows of kXcdWindow blocks.  Ranges over
             // the whole launch would set the XCDs 1/8 of the batch apart, at
             // equal places of equal rows, which for power-of-two strides are
-            // the same memory channels.)
-            const unsigned win = PREFETCH ? 0u : blockIdx.x / kXcdWindow * kXcdWindow;
+            // the same memory channels.  Where the data fits the L2s they are
+            // right: a transform then stays on one XCD from pass to pass.)
+            const bool whole = PREFETCH || a.near;
+            const unsigned win = whole ? 0u : blockIdx.x / kXcdWindow * kXcdWindow;
             const unsigned wb = blockIdx.x - win;
-            const unsigned wn =
-                PREFETCH ? (unsigned)G
-                         : ((unsigned)G - win < kXcdWindow ? (unsigned)G - win : kXcdWindow);
+            const unsigned wn = whole || (unsigned)G - win < kXcdWindow ? (unsigned)G - win
+                                                                        : kXcdWindow;
             const int off = (int)(win + (share ? xcd_tile(wb, wn) : wb));
             int grp = off;
             if constexpr (!PREFETCH) {  // one tile per block
