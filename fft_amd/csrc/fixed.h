@@ -23,6 +23,14 @@
 // lengths, FP64 1.05x of 112 up to 4860, real 1.13x forward and 1.17x inverse
 // of 98 (up to 2.0x), column passes 1.09x (first pass) and 1.19x (second) of
 // 38; the second at nearly every length above it (0.80-0.96x).
+// Blocks sized for the second schedule are too large for the first: two or
+// three per CU, each waiting for its own loads.  Between 30 and 130 MB a launch
+// that cost up to 25 % against the second, and lengths that lost 4 % or more
+// hold half as many transforms per block (FP64 64 MB, persistent / one group /
+// half: 400 24.4 / 30.5 / 26.3 us, 125 27.4 / 32.8 / 27.7, 75 29.5 / 32.1 / 24.4;
+// 128 MB: 47.7 / 50.5 / 44.3, 50.1 / 58.0 / 47.3, 47.7 / 52.5 / 43.7), those of one
+// transform per block other twiddle loads (Sched TW), or the second schedule
+// back (kPersist: FP32 7680, FP64 3240, 3600, 3840, 4320).
 #pragma once
 
 #include "stockham.h"
@@ -98,6 +106,8 @@ __device__ __forceinline__ void flip_im(C2<double> &x, uint32_t m) {
 //         (On the real 2048 pair of the bench step, non-temporal accesses in
 //         the forward kernel made it 10 % faster and the inverse leg that
 //         follows it 10 % slower, with no net gain; they are not used there.)
+//   TW    1 or 0: one-group kernels load a stage's twiddles before the exchange
+//         that feeds it, or after it (-1: as TW_EARLY below has it).
 constexpr int kLdsNoPad = 30;
 constexpr int kNoPrefetch = -100;  // PFS: never persistent
 constexpr int kPersist = 100;      // PFS + kPersist: persistent at any tile size
@@ -105,7 +115,7 @@ constexpr unsigned kXcdWindow = 256;  // blocks numbered XCD-contiguously togeth
 // Largest tile of which two blocks fit a CU.
 constexpr size_t kSharedCuLds = 80 * 1024;
 template <int PFS_, int MINW_, int PAIR_ = 1, int PF_FIRST_ = 0, int PADSH_ = kLdsPadShift,
-          int NT_ = 0>
+          int NT_ = 0, int TW_ = -1>
 struct Sched {
     static constexpr int PFS = PFS_;
     static constexpr int MINW = MINW_;
@@ -113,6 +123,7 @@ struct Sched {
     static constexpr int PF_FIRST = PF_FIRST_;
     static constexpr int PADSH = PADSH_;
     static constexpr int NT = NT_;
+    static constexpr int TW = TW_;
     static constexpr bool ROT = false;
 };
 // Column passes that also rotate (half-bin shifted real transforms): the
@@ -152,7 +163,8 @@ template <typename T_, int N, int TPT, int TPW, int MODE, class SCH, int... Rs>
 struct Fixed {
     using T = typename FixedElem<T_>::T;
     using ST = Storage<T, typename FixedElem<T_>::S>;
-    static constexpr int PFS = SCH::PFS >= kPersist ? SCH::PFS - kPersist : SCH::PFS;
+    static constexpr bool PERSIST = SCH::PFS > kPersist / 2;  // (PFS may be negative)
+    static constexpr int PFS = PERSIST ? SCH::PFS - kPersist : SCH::PFS;
     static constexpr int MINW = SCH::MINW;
     static constexpr int NST = sizeof...(Rs);
     static constexpr int RAD[NST] = {Rs...};
@@ -199,12 +211,14 @@ struct Fixed {
     // Persistent and pipelined only where one block fills a CU (see the top of
     // the file).
     static constexpr bool PREFETCH =
-        SCH::PFS != kNoPrefetch && (SCH::PFS >= kPersist || LDS_BYTES > kSharedCuLds);
+        SCH::PFS != kNoPrefetch && (PERSIST || LDS_BYTES > kSharedCuLds);
     // One group per block: a stage's twiddles are loaded before the exchange
     // that feeds it (FP32 column passes 1-3 % faster, FP64 ones 4-9 %, one 4096
-    // transform 5.4 -> 5.1 us; FP64 single passes, short of registers, would
-    // be up to 14 % slower).
-    static constexpr bool TW_EARLY = !PREFETCH && (sizeof(T) == 4 || COL);
+    // transform 5.4 -> 5.1 us; FP64 single passes in blocks of the persistent
+    // schedule's size, short of registers, would be up to 14 % slower, and those
+    // in blocks of half that are 1-5 % faster: their Sched says so).
+    static constexpr bool TW_EARLY =
+        !PREFETCH && (SCH::TW >= 0 ? SCH::TW == 1 : sizeof(T) == 4 || COL);
 
     static constexpr int ns_of(int s) {
         int p = 1;

@@ -8,6 +8,8 @@
 // with neither 3 % slower, batches of 128 MB:
 // median 1.44x over the runtime-planned pass (7500 178 -> 128 us); 300, 360, 450,
 // 675 and 768 lose 3-21 %.
+// (Half-size blocks, a twiddle choice, the seventh Sched value, or kPersist: lengths
+// that one group per block had slowed; figures at the top of fixed.h.)
 #include "fixed.h"
 
 namespace sfft {
@@ -27,7 +29,7 @@ const FixedC2C<X, 720, 48, 5, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 15, 3> c72
 const FixedC2C<X, 810, 90, 3, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 10, 9, 9> c810;
 const FixedC2C<X, 972, 108, 2, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 12, 9, 9> c972;
 const FixedC2C<X, 1152, 96, 3, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 12, 6> c1152;
-const FixedC2C<X, 1280, 86, 3, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 16, 5> c1280;
+const FixedC2C<X, 1280, 86, 2, Sched<0, 0, 0, 0, kLdsPadShift, 0, 1>, 0, 16, 16, 5> c1280;
 const FixedC2C<X, 1458, 162, 2, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 9, 9, 9, 2> c1458;
 const FixedC2C<X, 1620, 180, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 15, 12, 9> c1620;
 const FixedC2C<X, 1920, 128, 2, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 15, 8> c1920;

@@ -7,6 +7,8 @@
 // with neither 3 % slower, batches of 128 MB:
 // R2C forward and inverse median 1.31x, up to 2.4x (15000 133 + 142 -> 103 + 112
 // us); h = 360, 384, 450, 640, 675 and 768 lose up to 22 %.
+// (Half-size blocks, a twiddle choice, the seventh Sched value, or kPersist: lengths
+// that one group per block had slowed; figures at the top of fixed.h.)
 #include "fixed.h"
 
 namespace sfft {
@@ -14,7 +16,7 @@ namespace {
 const FixedReal<double, 90, 10, 26, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 10, 9> r180;
 const FixedReal<double, 144, 12, 21, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 12, 12> r288;
 const FixedReal<double, 225, 15, 17, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 15, 15> r450;
-const FixedReal<double, 320, 22, 12, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 5, 4> r640;
+const FixedReal<double, 320, 22, 6, Sched<0, 0, 0, 0, kLdsPadShift, 0, 1>, 0, 16, 5, 4> r640;
 const FixedReal<double, 500, 50, 5, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 10, 10, 5> r1000;
 const FixedReal<double, 729, 81, 3, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 9, 9, 9> r1458;
 const FixedReal<double, 1000, 100, 3, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 10, 10, 10> r2000;

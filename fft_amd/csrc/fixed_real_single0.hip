@@ -14,6 +14,8 @@
 //           Sched<prefetch stage, min waves per SIMD, pair loads, prefetch first,
 //           LDS pad shift>, variant, radices...>
 // (The rates were measured with persistent kernels.)
+// (Half-size blocks, a twiddle choice, the seventh Sched value, or kPersist: lengths
+// that one group per block had slowed; figures at the top of fixed.h.)
 #include "fixed.h"
 
 namespace sfft {
@@ -27,10 +29,10 @@ const FixedReal<float, 640, 43, 5, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 8, 5>
 const FixedReal<float, 768, 52, 4, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 16, 3> r1536;  // 3527 / 3309 -> 3778 / 3801
 const FixedReal<float, 960, 64, 4, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 15, 4> r1920;  // 4055 / 4007 -> 4272 / 4201
 const FixedReal<float, 1152, 96, 2, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 12, 6> r2304;  // 3807 / 3654 -> 4127 / 4331
-const FixedReal<float, 1296, 144, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 12, 12, 9> r2592;  // 2833 / 2742 -> 3649 / 3579
+const FixedReal<float, 1296, 144, 1, Sched<0, 0, 0, 0, kLdsPadShift, 0, 0>, 0, 12, 12, 9> r2592;  // 2833 / 2742 -> 3649 / 3579
 const FixedReal<float, 1536, 128, 2, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 16, 6> r3072;  // 3786 / 3744 -> 4143 / 4109
 const FixedReal<float, 2250, 225, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 15, 15, 10> r4500;  // 3173 / 2923 -> 3303 / 3281
-const FixedReal<float, 2560, 256, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 16, 10> r5120;  // 3607 / 3492 -> 4100 / 4215
+const FixedReal<float, 2560, 256, 1, Sched<0, 0, 0, 0, kLdsPadShift, 0, 0>, 0, 16, 16, 10> r5120;  // 3607 / 3492 -> 4100 / 4215
 const FixedReal<float, 3072, 256, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 16, 12> r6144;  // 3924 / 3792 -> 4305 / 4067
 const FixedReal<float, 3888, 432, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 12, 9, 6, 6> r7776;  // 2360 / 2168 -> 3045 / 2210
 const FixedReal<float, 4500, 300, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 15, 15, 5, 4> r9000;  // 2171 / 2055 -> 2374 / 2131

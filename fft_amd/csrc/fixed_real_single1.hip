@@ -14,6 +14,8 @@
 //           Sched<prefetch stage, min waves per SIMD, pair loads, prefetch first,
 //           LDS pad shift>, variant, radices...>
 // (The rates were measured with persistent kernels.)
+// (Half-size blocks, a twiddle choice, the seventh Sched value, or kPersist: lengths
+// that one group per block had slowed; figures at the top of fixed.h.)
 #include "fixed.h"
 
 namespace sfft {
@@ -24,7 +26,7 @@ const FixedReal<float, 300, 13, 19, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 25, 12> 
 const FixedReal<float, 405, 45, 5, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 9, 9, 5> r810;  // 3419 / 3079 -> 4603 / 3859
 const FixedReal<float, 500, 50, 5, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 10, 10, 5> r1000;  // 3898 / 3338 -> 4652 / 4090
 const FixedReal<float, 648, 72, 3, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 12, 9, 6> r1296;  // 3120 / 2982 -> 4063 / 3574
-const FixedReal<float, 800, 32, 8, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 32, 25> r1600;  // 3726 / 3622 -> 4075 / 4036
+const FixedReal<float, 800, 32, 4, Sched<0, 0, 0, 0, kLdsPadShift, 0, 0>, 0, 32, 25> r1600;  // 3726 / 3622 -> 4075 / 4036
 const FixedReal<float, 972, 108, 2, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 12, 9, 9> r1944;  // 3346 / 3094 -> 4109 / 3900
 const FixedReal<float, 1200, 80, 3, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 15, 5> r2400;  // 3898 / 3830 -> 4246 / 4166
 const FixedReal<float, 1440, 144, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 12, 12, 10> r2880;  // 3020 / 2915 -> 3907 / 3810

@@ -16,6 +16,8 @@
 // (The rates were measured with persistent kernels; lines with kPersist keep
 // that schedule, 4-20 % faster there than one group per block, and lines with
 // kNoPrefetch the latter above 80 KB of LDS, 7-50 % faster.)
+// (Half-size blocks, a twiddle choice, the seventh Sched value, or kPersist: lengths
+// that one group per block had slowed; figures at the top of fixed.h.)
 #include "fixed.h"
 
 namespace sfft {
@@ -31,7 +33,7 @@ const FixedReal<float, 1000, 100, 2, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 10, 10,
 const FixedReal<float, 1215, 135, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 15, 9, 9> r2430;  // 2602 / 2541 -> 3145 / 2971
 const FixedReal<float, 1458, 162, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 9, 9, 9, 2> r2916;  // 2531 / 2465 -> 3615 / 3152
 const FixedReal<float, 1944, 216, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 9, 6, 6, 6> r3888;  // 2618 / 2530 -> 3651 / 2978
-const FixedReal<float, 2400, 240, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 15, 10> r4800;  // 3451 / 3383 -> 3910 / 3756
+const FixedReal<float, 2400, 240, 1, Sched<0, 0, 0, 0, kLdsPadShift, 0, 0>, 0, 16, 15, 10> r4800;  // 3451 / 3383 -> 3910 / 3756
 const FixedReal<float, 2880, 240, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 15, 12> r5760;  // 3835 / 3577 -> 3961 / 3912
 const FixedReal<float, 3456, 288, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 6, 6, 6> r6912;  // 1987 / 1984 -> 2744 / 2158
 const FixedReal<float, 4050, 338, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 15, 15, 6, 3> r8100;  // 2104 / 1903 -> 2337 / 1970

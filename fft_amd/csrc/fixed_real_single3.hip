@@ -16,6 +16,8 @@
 // (The rates were measured with persistent kernels; lines with kPersist keep
 // that schedule, 4-20 % faster there than one group per block, and lines with
 // kNoPrefetch the latter above 80 KB of LDS, 7-50 % faster.)
+// (Half-size blocks, a twiddle choice, the seventh Sched value, or kPersist: lengths
+// that one group per block had slowed; figures at the top of fixed.h.)
 #include "fixed.h"
 
 namespace sfft {
@@ -30,7 +32,7 @@ const FixedReal<float, 864, 72, 3, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 12, 12, 6
 const FixedReal<float, 1080, 90, 2, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 15, 12, 6> r2160;  // 3539 / 3290 -> 3824 / 3530
 const FixedReal<float, 1280, 86, 2, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 16, 5> r2560;  // 3747 / 3598 -> 4090 / 4138
 const FixedReal<float, 1500, 150, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 15, 10, 10> r3000;  // 2983 / 2824 -> 3544 / 3104
-const FixedReal<float, 2187, 243, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 9, 9, 9, 3> r4374;  // 2987 / 2754 -> 4027 / 3726
+const FixedReal<float, 2187, 243, 1, Sched<0, 0, 0, 0, kLdsPadShift, 0, 0>, 0, 9, 9, 9, 3> r4374;  // 2987 / 2754 -> 4027 / 3726
 const FixedReal<float, 2430, 270, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 10, 9, 9, 3> r4860;  // 1683 / 1608 -> 2404 / 1799
 const FixedReal<float, 2916, 324, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 9, 9, 6, 6> r5832;  // 1960 / 1817 -> 2706 / 1919
 const FixedReal<float, 3645, 405, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 9, 9, 9, 5> r7290;  // 2375 / 2138 -> 3212 / 2463

@@ -16,11 +16,13 @@
 //          Sched<prefetch stage, min waves per SIMD, pair loads, prefetch first,
 //          LDS pad shift>, variant, radices...>
 // (The rates were measured with persistent kernels.)
+// (Half-size blocks, a twiddle choice, the seventh Sched value, or kPersist: lengths
+// that one group per block had slowed; figures at the top of fixed.h.)
 #include "fixed.h"
 
 namespace sfft {
 namespace {
-const FixedC2C<float, 162, 18, 14, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 9, 9, 2> c162;  // 4076 -> 4777
+const FixedC2C<float, 162, 18, 7, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 9, 9, 2> c162;  // 4076 -> 4777
 const FixedC2C<float, 288, 24, 10, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 12, 12, 2> c288;  // 4478 -> 4880
 const FixedC2C<float, 405, 45, 5, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 9, 9, 5> c405;  // 4007 -> 4673
 const FixedC2C<float, 576, 48, 5, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 6, 6> c576;  // 4426 -> 4888
@@ -38,7 +40,7 @@ const FixedC2C<float, 5120, 171, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 32, 32, 
 const FixedC2C<float, 5760, 240, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 32, 15, 12> c5760;  // 3084 -> 4608
 const FixedC2C<float, 6144, 205, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 32, 32, 6> c6144;  // 3192 -> 4298
 const FixedC2C<float, 6561, 729, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 9, 9, 9, 9> c6561;  // 2575 -> 4060
-const FixedC2C<float, 7680, 256, 1, Sched<0, 0, 0, 0, kLdsPadShift, 3>, 0, 32, 16, 15> c7680;  // 3422 -> 4318
+const FixedC2C<float, 7680, 256, 1, Sched<kPersist, 0, 0, 0, kLdsPadShift, 3>, 0, 32, 16, 15> c7680;  // 3422 -> 4318
 const FixedC2C<float, 8640, 720, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 12, 12, 12, 5> c8640;  // 2257 -> 3813
 const FixedC2C<float, 10000, 1000, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 10, 10, 10, 10> c10000;  // 2554 -> 3956
 const FixedC2C<float, 10800, 720, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 16, 15, 15, 3> c10800;  // 2486 -> 3622
