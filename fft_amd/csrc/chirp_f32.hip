@@ -2,11 +2,15 @@
 // to 4096.  ChirpReg<type, rows of a longer one, M, threads per transform,
 // transforms per block, minimum waves per SIMD, radices...>: mostly R b R
 // with M / R threads, one radix-R butterfly each.  These kernels are bound by vector
-// instructions (about 100 per element of M), so a length is listed only where
-// it beat the next power of two: 1280, 1792, 2560 and 3840 did not (6.2 to 9.7
-// ps per element of M against 4.9 at 1024 and 2048, at 8 to 16 transforms
-// resident per CU).  Two transforms per thread, which halves the table loads,
-// measured 0.62-0.98x: half the resident waves.
+// instructions (about 100 per element of M).  The lengths between the powers of
+// two are those that beat the next one when all took sixteen elements a thread
+// (1280, 1792, 2560 and 3840 did not).  Against the eight of 512 to 4096 now,
+// both directions, 1 / 512 / 4096 transforms, this length / the next power of
+// two: 448 (n = 223) 11.1 / 10.1, 12.9 / 11.5, 21.1 / 19.3 us, 1536 (n = 761)
+// 17.3 / 11.0, 19.5 / 14.4, 71.1 / 60.8 (but 31.4 / 34.0 at 2048), so these two
+// would go; 768 and 3072 take a third more than 1024 and 4096 for one transform
+// and 6 to 15 % less for 4096.  Two transforms per thread, which halves the table
+// loads, measured 0.62-0.98x: half the resident waves.
 // 1024, 2048 and 4096 take eight elements a thread and one more stage, which
 // halves a wave's registers and LDS (twice the waves).  Both directions, sixteen
 // / eight: 509 x 8192 68.2 / 64.8 us, 1009 x 4096 73.4 / 68.2, x 20000 376 / 321,

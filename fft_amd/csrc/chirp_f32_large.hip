@@ -2,7 +2,9 @@
 // lengths 5120...16384, one transform per block, 8 to 16 elements a thread so
 // that a CU holds 16 waves or more.  Three stages of radix 32 b 32 (32 elements
 // a thread, two waves per SIMD) were slower: M = 5120 105 -> 81 us, 8192 58 ->
-// 49, 16384 89 -> 78.  12288 and 15360 lose to 16384.
+// 49, 16384 89 -> 78.  12288 and 15360 lose to 16384, and so does 10240 (n =
+// 5003, both directions, 1 / 512 / 4096 transforms: 40.1 / 36.9, 108.6 / 87.6,
+// 911 / 671 us), which would go too.
 #include "chirp.h"
 
 namespace sfft {
