@@ -18,6 +18,9 @@
 // (The rates were measured with persistent kernels; lines with kPersist keep
 // that schedule, 4-20 % faster there than one group per block, and lines with
 // kNoPrefetch the latter above 80 KB of LDS, 7-50 % faster.)
+// 800 has the stores only (a schedule that ends in 2): in the one-group schedule
+// non-temporal loads cost it 17 % at 32 MB (persistent 13.4 us, 15.7, with stores
+// only 13.9) and with cold inputs gain nothing (126 MB 53.5 and 53.6 us).
 // (Half-size blocks, a twiddle choice, the seventh Sched value, or kPersist: lengths
 // that one group per block had slowed; figures at the top of fixed.h.)
 #include "fixed.h"
@@ -28,7 +31,7 @@ const FixedC2C<float, 125, 9, 28, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 25, 5> c12
 const FixedC2C<float, 270, 23, 11, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 15, 6, 3> c270;  // 4145 -> 4464
 const FixedC2C<float, 384, 16, 16, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 32, 12> c384;  // 4657 -> 4974
 const FixedC2C<float, 540, 45, 5, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 15, 6, 6> c540;  // 4116 -> 4361
-const FixedC2C<float, 800, 32, 8, Sched<0, 0, 0, 0, kLdsPadShift, 3>, 0, 32, 25> c800;  // 4328 -> 4811
+const FixedC2C<float, 800, 32, 8, Sched<0, 0, 0, 0, kLdsPadShift, 2>, 0, 32, 25> c800;  // 4328 -> 4811
 const FixedC2C<float, 1000, 100, 2, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 10, 10, 10> c1000;  // 4081 -> 4604
 const FixedC2C<float, 1440, 144, 1, Sched<0, 0, 0, 0, kLdsPadShift>, 0, 12, 12, 10> c1440;  // 3897 -> 4952
 const FixedC2C<float, 1600, 54, 2, Sched<0, 0, 0, 0, kLdsPadShift, 0, 0>, 0, 32, 10, 5> c1600;  // 4194 -> 4438
