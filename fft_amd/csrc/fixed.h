@@ -967,12 +967,12 @@ struct FixedC2C {
 };
 
 // Registers the real forward / inverse pair of one compile-time plan of the
-// half-length complex core N (real length 2N).
-template <typename T, int N, int TPT, int TPW, class SCH, int VARIANT, int... Rs>
-struct FixedReal {
-    using FR = Fixed<T, N, TPT, TPW, kModeR2C, SCH, Rs...>;
-    using FI = Fixed<T, N, TPT, TPW, kModeC2R, SCH, Rs...>;
-    FixedReal() {
+// half-length complex core N (real length 2N), SF and SI the schedules of the two.
+template <typename T, int N, int TPT, int TPW, class SF, class SI, int VARIANT, int... Rs>
+struct FixedRealOf {
+    using FR = Fixed<T, N, TPT, TPW, kModeR2C, SF, Rs...>;
+    using FI = Fixed<T, N, TPT, TPW, kModeC2R, SI, Rs...>;
+    FixedRealOf() {
         FixedKernel k{};
         k.n = N;
         k.variant = VARIANT;
@@ -992,6 +992,9 @@ struct FixedReal {
         register_fixed(k);
     }
 };
+
+template <typename T, int N, int TPT, int TPW, class SCH, int VARIANT, int... Rs>
+using FixedReal = FixedRealOf<T, N, TPT, TPW, SCH, SCH, VARIANT, Rs...>;
 
 // Registers the column passes of one compile-time plan of column length N
 // (registry kind 2): the first pass of a two-pass plan (kModeColRow, WR columns

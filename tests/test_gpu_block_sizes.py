@@ -15,13 +15,13 @@ pytestmark = pytest.mark.gpu
 TOL = {L.F32: 1e-6, L.F64: 1e-12, L.F32X: 1e-7}
 REAL = (L.R2C, L.R2C_HALFSHIFT)
 CASES = (
-    [(L.C2C, L.F32, n) for n in (162, 256, 512, 648, 1600, 2048, 7680)]
+    [(L.C2C, L.F32, n) for n in (162, 256, 512, 648, 800, 1600, 2048, 7680)]
     + [(L.C2C, L.F64, n) for n in (75, 90, 125, 162, 200, 225, 256, 288, 375, 384, 400, 405, 480,
                                    500, 512, 640, 720, 810, 960, 972, 1024, 1080, 1125, 1200,
                                    1250, 1728, 1920, 2048, 2160, 2187, 2500, 3000, 3125, 3240,
                                    3375, 3600, 3840, 4320)]
     + [(L.C2C, L.F32X, 1280)]
-    + [(k, L.F32, 2 * h) for k in REAL for h in (512, 800, 1296, 2187, 2400, 2560)]
+    + [(k, L.F32, 2 * h) for k in REAL for h in (512, 800, 1296, 2187, 2400, 2560, 6480)]
     + [(k, L.F64, 2 * h) for k in REAL for h in (300, 320, 1280, 2048)])
 
 
